@@ -16,22 +16,26 @@ constexpr double kEulerGamma = 0.57721566490153286061;
 constexpr double kQuarterPi = 0.78539816339744830962;
 constexpr double kLn2 = 0.69314718055994530942;
 
-// 1/x in FP64: v_rcp_f64 estimate + two Newton steps (error ~1 ulp).
+// 1/x in FP64: v_rcp_f64 estimate r with e = 1 - x r (measured |e| <=
+// 2^-24.4 over [1e-8, 1e4]) and one third-order step 1/x = r (1 + e + e^2 +
+// O(e^3)), the remainder 2^-73: three operations, where two Newton steps to
+// the same result are four.
 __device__ __forceinline__ double rcp64(double x) {
-    double r = __builtin_amdgcn_rcp(x);
-    double e = __builtin_fma(-x, r, 1.0);
-    r = __builtin_fma(r, e, r);
-    e = __builtin_fma(-x, r, 1.0);
-    return __builtin_fma(r, e, r);
+    const double r = __builtin_amdgcn_rcp(x);
+    const double e = __builtin_fma(-x, r, 1.0);
+    return __builtin_fma(r, __builtin_fma(e, e, e), r);
 }
 
-// 1/sqrt(x) in FP64: v_rsq_f64 estimate + two Newton steps.
+// 1/sqrt(x) in FP64: v_rsq_f64 estimate y with h = 1 - x y^2 (measured
+// |h| <= 2^-23.2) and one third-order step 1/sqrt(x) = y (1 + h/2 + 3 h^2/8 +
+// O(h^3)), the remainder 2^-71: five operations in the place of the eight of
+// two Newton steps, which the FP64 pair kernels (bound by FP64 issue) feel:
+// 3D Laplace SL symmetric sum at 122,880 nodes 4.97 -> 4.22 ms, 3D Helmholtz
+// combined field at 12,000 nodes 0.267 -> 0.258 ms.
 __device__ __forceinline__ double rsq64(double x) {
-    double y = __builtin_amdgcn_rsq(x);
-    double h = __builtin_fma(-(x * y), y, 1.0);
-    y = __builtin_fma(0.5 * y, h, y);
-    h = __builtin_fma(-(x * y), y, 1.0);
-    return __builtin_fma(0.5 * y, h, y);
+    const double y = __builtin_amdgcn_rsq(x);
+    const double h = __builtin_fma(-(x * y), y, 1.0);
+    return __builtin_fma(y * h, __builtin_fma(h, 0.375, 0.5), y);
 }
 
 // FP32 hardware estimate refined once in FP64: ~1e-14 relative, enough for
