@@ -894,24 +894,15 @@ static int adjoint_sigma_only(Op *op, const double *ubar, double *sigma_bar) {
     int kind = op->kind;
     const KParams kp = op_params(op, &kind);
 
-    // symmetric plan: tiles of 256 in groups of G
     SymFn fsym = nullptr;
-    int64_t T = (n + kSymBS - 1) / kSymBS, S = 0;
-    if (op->trg == op->src && op->sym && kind < INTI_FF_SL && T >= 2 &&
-        (op->sym == 2 || T * (T + 1) / 2 >= 2LL * ctx->num_cu)) {
-        int G = 0;
-        for (int g : {1, 2, 4}) {
-            if (op->sym_group && g != op->sym_group) continue;
-            S = (T + g - 1) / g;
-            if ((size_t)S * (size_t)n * cw * sizeof(double) <= kAdjSymMaxBytes) {
-                G = g;
-                break;
-            }
-        }
-        if (G && op->pde == INTI_LAPLACE && op->dim == 2) fsym = sym_trans_pick_lap2(kind, G);
-        if (G && op->pde == INTI_LAPLACE && op->dim == 3) fsym = sym_trans_pick_lap3(kind, G);
-        if (G && op->pde == INTI_HELMHOLTZ && op->dim == 2) fsym = sym_trans_pick_helm2(kind, G);
-        if (G && op->pde == INTI_HELMHOLTZ && op->dim == 3) fsym = sym_trans_pick_helm3(kind, G);
+    SymPlan sp{};
+    int64_t S = 0;
+    if (plan_sym(op, kind, sp)) {
+        S = sp.S;
+        if (op->pde == INTI_LAPLACE && op->dim == 2) fsym = sym_trans_pick_lap2(kind, sp.tile, sp.G);
+        if (op->pde == INTI_LAPLACE && op->dim == 3) fsym = sym_trans_pick_lap3(kind, sp.tile, sp.G);
+        if (op->pde == INTI_HELMHOLTZ && op->dim == 2) fsym = sym_trans_pick_helm2(kind, sp.tile, sp.G);
+        if (op->pde == INTI_HELMHOLTZ && op->dim == 3) fsym = sym_trans_pick_helm3(kind, sp.tile, sp.G);
     }
     // one-direction plan: the sum's targets are the n sources (tiles of
     // 256), its sources the m targets cut into `split` chunks
@@ -954,7 +945,7 @@ static int adjoint_sigma_only(Op *op, const double *ubar, double *sigma_bar) {
         a.xy = op->src->coords; a.nrm = op->src->normals; a.w = nullptr;
         a.x = xc;
         a.part = (double *)dpart.p;
-        a.ntiles = T; a.ngroups = S;
+        a.ntiles = sp.T; a.ngroups = S;
         a.distinct = op->src->distinct ? 1 : 0;
         a.ch_ik = 0;  // the transposed sums are FP64 (no staged ch q)
         a.p = kp;

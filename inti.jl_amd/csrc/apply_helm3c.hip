@@ -10,4 +10,5 @@ ApplyFn apply_pick_helm3c(int kind, int nr) {
     if (nr == 16) return apply_kind<kHelmCK, 3, false, 16>(kind);
     return nullptr;
 }
+RowFn row_pick_helm3c(int kind) { return row_kind<kHelmCK, 3, false>(kind); }
 }  // namespace inti

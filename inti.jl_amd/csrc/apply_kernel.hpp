@@ -412,6 +412,142 @@ __global__ __launch_bounds__(apply_threads<NR>()) void k_apply(ApplyArgs a) {
     apply_any<PDE, DIM, KIND, MIXED, NR, TRANS>(a, b % a.split, b / a.split, s_geo, s_q);
 }
 
+// ------------------------------------------------------------- epilogue
+struct ReduceArgs {
+    int64_t m;
+    int split;
+    const double *part;  // nr x split x m
+    int64_t ldx, ldy;    // leading dimensions of x and y (elements)
+    const int32_t *rowptr;
+    const int32_t *colind;
+    const double *cval;
+    const double *x;  // density (for the correction and identity terms)
+    double *y;
+    double ar, ai, br, bi, cr, ci;
+    double pr, pi;  // post factor of the direct sum
+    int beta_zero;
+    int has_id;
+};
+
+// y_i = alpha * (post * (sr + i si) + (dA x)_i + cid x_i) + beta * y_i
+template <bool CPLX>
+__device__ __forceinline__ void reduce_epilogue(const ReduceArgs &a, int64_t i, const double *x, double *y,
+                                                double sr, double si) {
+    {
+        const double tr = a.pr * sr - a.pi * si, ti = a.pr * si + a.pi * sr;
+        sr = tr;
+        si = ti;
+    }
+    if (a.rowptr) {
+        const int32_t p0 = a.rowptr[i], p1 = a.rowptr[i + 1];
+        for (int32_t p = p0; p < p1; ++p) {
+            const int32_t j = a.colind[p];
+            if constexpr (CPLX) {
+                const double vr = a.cval[2 * p], vi = a.cval[2 * p + 1];
+                const double xr = x[2 * j], xi = x[2 * j + 1];
+                sr += vr * xr - vi * xi;
+                si += vr * xi + vi * xr;
+            } else {
+                sr += a.cval[p] * x[j];
+            }
+        }
+    }
+    if (a.has_id) {
+        if constexpr (CPLX) {
+            const double xr = x[2 * i], xi = x[2 * i + 1];
+            sr += a.cr * xr - a.ci * xi;
+            si += a.cr * xi + a.ci * xr;
+        } else {
+            sr += a.cr * x[i];
+        }
+    }
+    if constexpr (CPLX) {
+        double yr = a.ar * sr - a.ai * si, yi = a.ar * si + a.ai * sr;
+        if (!a.beta_zero) {
+            const double or_ = y[2 * i], oi = y[2 * i + 1];
+            yr += a.br * or_ - a.bi * oi;
+            yi += a.br * oi + a.bi * or_;
+        }
+        y[2 * i] = yr;
+        y[2 * i + 1] = yi;
+    } else {
+        double yr = a.ar * sr;
+        if (!a.beta_zero) yr += a.br * y[i];
+        y[i] = yr;
+    }
+}
+
+// ------------------------------------------------------ small sums, one launch
+// One right-hand side of few targets in one launch: a block takes tb targets
+// (4 ... 64, a power of two) and 256 / tb threads share each target's
+// sources, thread t of a target taking sources t, t + 256 / tb, ... read
+// straight from memory (consecutive threads read consecutive sources). The
+// threads' sums are added in a fixed order (lanes by a butterfly, then the
+// four waves in wave order) and the block finishes its rows itself (post
+// factor, correction, identity, alpha / beta): no partial sums and no second
+// kernel. See launch_apply for where it is taken.
+struct RowArgs {
+    ApplyArgs s;
+    ReduceArgs e;
+    int tb;
+};
+
+template <int PDE, int DIM, int KIND, bool MIXED>
+__global__ __launch_bounds__(kApplyBS) void k_apply_row(RowArgs a) {
+    constexpr bool CPLX = PDE != INTI_LAPLACE;
+    constexpr int NW = kApplyBS / 64;
+    __shared__ double2 s_w[NW][64];
+    const ApplyArgs &g = a.s;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tb = a.tb, t = tid & (tb - 1), nsl = kApplyBS / tb;
+    const int64_t i = (int64_t)blockIdx.x * tb + t;
+    const int64_t ic = i < g.m ? i : g.m - 1;
+    double xt[DIM], nt[DIM];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) {
+        xt[d] = g.tx[d * g.tstride + ic];
+        nt[d] = g.tn ? g.tn[d * g.tstride + ic] : 0.0;
+    }
+    double sr = 0.0, si = 0.0;
+    constexpr int UNR = CPLX && DIM == 2 ? 1 : 2;
+#pragma unroll UNR
+    for (int64_t j = tid / tb; j < g.n; j += nsl) {
+        double y[DIM], ny[DIM];
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+            y[d] = g.sx[d * g.sstride + j];
+            ny[d] = g.sn ? g.sn[d * g.sstride + j] : 0.0;
+        }
+        const double w = g.sw[j];
+        double kr, ki;
+        pair_raw_xy<PDE, DIM, KIND, MIXED>(xt, nt, y, ny, g.p, kr, ki);
+        if constexpr (CPLX) {
+            const double2 xv = reinterpret_cast<const double2 *>(g.x)[j];
+            const double qr = w * xv.x, qi = w * xv.y;
+            sr = __builtin_fma(kr, qr, sr);
+            sr = __builtin_fma(-ki, qi, sr);
+            si = __builtin_fma(kr, qi, si);
+            si = __builtin_fma(ki, qr, si);
+        } else {
+            sr = __builtin_fma(kr, w * g.x[j], sr);
+        }
+    }
+    for (int o = tb; o < 64; o *= 2) {
+        sr += __shfl_xor(sr, o);
+        if constexpr (CPLX) si += __shfl_xor(si, o);
+    }
+    if (lane < tb) s_w[wave][lane] = make_double2(sr, si);
+    __syncthreads();
+    if (tid < tb && i < g.m) {
+#pragma unroll
+        for (int w = 1; w < NW; ++w) {
+            sr += s_w[w][tid].x;
+            si += s_w[w][tid].y;
+        }
+        reduce_epilogue<CPLX>(a.e, i, a.e.x, a.e.y, sr, si);
+    }
+}
+
 // ------------------------------------------------------------ batched apply
 // Many independent problems (block-diagonal operator) in one persistent
 // launch: the work list holds (problem, target tile, source chunk) items,
@@ -479,6 +615,38 @@ static int apply_launcher(const ApplyArgs *a, dim3 grid, hipStream_t s) {
     }
     hipLaunchKernelGGL((k_apply<PDE, DIM, KIND, MIXED, NR, TRANS>), grid, dim3(apply_threads<NR>()), 0, s, *a);
     return 0;
+}
+
+using RowFn = void (*)(const RowArgs &, dim3, hipStream_t);
+
+template <int PDE, int DIM, int KIND, bool MIXED>
+static void row_launcher(const RowArgs &a, dim3 grid, hipStream_t s) {
+    hipLaunchKernelGGL((k_apply_row<PDE, DIM, KIND, MIXED>), grid, dim3(kApplyBS), 0, s, a);
+}
+
+template <int PDE, int DIM, bool MIXED>
+static RowFn row_kind(int kind) {
+    switch (kind) {
+        case INTI_SL: return row_launcher<PDE, DIM, INTI_SL, MIXED>;
+        case INTI_DL: return row_launcher<PDE, DIM, INTI_DL, MIXED>;
+        case INTI_ADL: return row_launcher<PDE, DIM, INTI_ADL, MIXED>;
+        case INTI_HS: return row_launcher<PDE, DIM, INTI_HS, MIXED>;
+        case INTI_COMB_SD: return row_launcher<PDE, DIM, INTI_COMB_SD, MIXED>;
+        case INTI_COMB_AH: return row_launcher<PDE, DIM, INTI_COMB_AH, MIXED>;
+    }
+    if constexpr (PDE == INTI_HELMHOLTZ) {
+        switch (kind) {
+            case INTI_FF_SL: return row_launcher<PDE, DIM, INTI_FF_SL, MIXED>;
+            case INTI_FF_DL: return row_launcher<PDE, DIM, INTI_FF_DL, MIXED>;
+            case INTI_FF_COMB: return row_launcher<PDE, DIM, INTI_FF_COMB, MIXED>;
+        }
+    }
+    return nullptr;
+}
+
+template <int PDE, int DIM>
+static RowFn row_pick_pd(int kind, int mixed) {
+    return mixed ? row_kind<PDE, DIM, true>(kind) : row_kind<PDE, DIM, false>(kind);
 }
 
 // transposed FP64 sums (one right-hand side) of the kinds with a pullback
@@ -581,5 +749,11 @@ ApplyFn apply_pick_lap3(int kind, int mixed, int nr);
 ApplyFn apply_pick_helm2(int kind, int mixed, int nr);
 ApplyFn apply_pick_helm3(int kind, int mixed, int nr);
 ApplyFn apply_pick_helm3c(int kind, int nr);  // complex wavenumber, FP64
+
+RowFn row_pick_lap2(int kind, int mixed);
+RowFn row_pick_lap3(int kind, int mixed);
+RowFn row_pick_helm2(int kind, int mixed);
+RowFn row_pick_helm3(int kind, int mixed);
+RowFn row_pick_helm3c(int kind);  // complex wavenumber, FP64
 
 }  // namespace inti

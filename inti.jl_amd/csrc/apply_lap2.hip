@@ -4,8 +4,9 @@
 
 namespace inti {
 ApplyFn apply_pick_lap2(int kind, int mixed, int nr) { return apply_pick_pd<INTI_LAPLACE, 2>(kind, mixed, nr); }
+RowFn row_pick_lap2(int kind, int mixed) { return row_pick_pd<INTI_LAPLACE, 2>(kind, mixed); }
 BatchFn batch_pick_lap2(int kind, int mixed, int nr) { return batch_pick_pd<INTI_LAPLACE, 2>(kind, mixed, nr); }
-SymFn sym_pick_lap2(int kind, int mixed, int G) { return sym_pick_pd<INTI_LAPLACE, 2>(kind, mixed, G); }
-SymFn sym_trans_pick_lap2(int kind, int G) { return sym_trans_pick_pd<INTI_LAPLACE, 2>(kind, G); }
+SymFn sym_pick_lap2(int kind, int mixed, int tile, int G) { return sym_pick_pd<INTI_LAPLACE, 2>(kind, mixed, tile, G); }
+SymFn sym_trans_pick_lap2(int kind, int tile, int G) { return sym_trans_pick_pd<INTI_LAPLACE, 2>(kind, tile, G); }
 ApplyFn apply_trans_pick_lap2(int kind) { return apply_trans_pick_pd<INTI_LAPLACE, 2>(kind); }
 }  // namespace inti

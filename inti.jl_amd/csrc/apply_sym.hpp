@@ -5,8 +5,8 @@
 // therefore evaluated once and applied in both directions (the shared parts
 // are common subexpressions of the two pair evaluations below).
 //
-// Work decomposition. The n nodes are cut into T tiles of 256 and the tiles
-// into S groups of G. Block (a, b), a <= b, takes the target tiles of group a
+// Work decomposition. The n nodes are cut into T tiles of 256 (smaller sums:
+// 128 or 64, one wave each, plan_sym) and the tiles into S groups of G. Block (a, b), a <= b, takes the target tiles of group a
 // against the source tiles of group b (within a diagonal block, the tile
 // pairs I <= J only). A wave holds 64 x TPL targets (TPL = 1, 2 or 4 per lane).
 // For each 64-source sub-tile, lane l at step s < 32 pairs its targets with
@@ -45,7 +45,17 @@ struct SymArgs {
     KParams p;
 };
 
-constexpr int kSymBS = 256;
+constexpr int kSymBS = 256;  // the largest tile
+
+// Tiles of a symmetric sum: `tile` nodes each, T of them in S groups of G
+// (64- and 128-node tiles: G = 1).
+struct SymPlan {
+    int tile, G;
+    int64_t T, S;
+};
+// The plan of a single-right-hand-side symmetric sum of op (kind: the kind
+// evaluated); false if it does not apply.
+bool plan_sym(const Op *op, int kind, SymPlan &P);
 
 // (a, b), a <= b, of block L in the row-major upper triangle of S x S.
 __device__ __forceinline__ void sym_item(int64_t L, int64_t S, int64_t &a, int64_t &b) {
@@ -105,7 +115,8 @@ struct SymRec {
     static constexpr int NF = DIM + (NRM ? DIM : 0) + (CPLX ? 2 : 1);
     static constexpr int NS = (NF + 1) / 2;
 
-    __device__ static __forceinline__ void put(double2 (*s)[kSymBS], int j, const double *y,
+    template <int TS>
+    __device__ static __forceinline__ void put(double2 (*s)[TS], int j, const double *y,
                                                const double *nv, double qr, double qi) {
         double f[2 * NS];
         int c = 0;
@@ -121,7 +132,8 @@ struct SymRec {
 #pragma unroll
         for (int k = 0; k < NS; ++k) s[k][j] = make_double2(f[2 * k], f[2 * k + 1]);
     }
-    __device__ static __forceinline__ void get(const double2 (*s)[kSymBS], int j, double *y,
+    template <int TS>
+    __device__ static __forceinline__ void get(const double2 (*s)[TS], int j, double *y,
                                                double *nv, double &qr, double &qi) {
         double f[2 * NS];
 #pragma unroll
@@ -155,7 +167,8 @@ struct SymRecF {
     static constexpr int NS = 4;
     // y (FP64), the normal in FP32 (it only enters the FP32 amplitudes) and
     // the FP32 source terms: y0 y1 | y2 n0 n1 | n2 cr ci - | qr qi kqi mkqr
-    __device__ static __forceinline__ void put(double2 (*s)[kSymBS], int j, const double *y, const double *nv,
+    template <int TS>
+    __device__ static __forceinline__ void put(double2 (*s)[TS], int j, const double *y, const double *nv,
                                                const QExt32 &q) {
         s[0][j] = make_double2(y[0], y[1]);
         s[1][j].x = y[2];
@@ -164,7 +177,8 @@ struct SymRecF {
             make_float4((float)nv[2], CHIK ? 0.0f : q.cr, CHIK ? 0.0f : q.ci, 0.0f);
         *reinterpret_cast<float4 *>(&s[3][j]) = make_float4(q.qr, q.qi, q.kqi, q.mkqr);
     }
-    __device__ static __forceinline__ void get(const double2 (*s)[kSymBS], int j, double *y, float *nv,
+    template <int TS>
+    __device__ static __forceinline__ void get(const double2 (*s)[TS], int j, double *y, float *nv,
                                                QExt32 &q) {
         const double2 v0 = s[0][j], v1 = s[1][j];
         const float2 n01 = *reinterpret_cast<const float2 *>(&v1.y);
@@ -181,7 +195,8 @@ struct SymRecF {
             q.ci = g.z;
         }
     }
-    __device__ static __forceinline__ void get(const double2 (*s)[kSymBS], int j, double *y, double *nv,
+    template <int TS>
+    __device__ static __forceinline__ void get(const double2 (*s)[TS], int j, double *y, double *nv,
                                                QExt32 &q) {
         float n32[3];
         get(s, j, y, n32, q);
@@ -194,8 +209,8 @@ struct SymRecF {
 // holds targets t, t + 256 / TPL, ...
 // TRANS: the transposed sum z_j = sum_i K(x_i, x_j) q_i (the kernel matrix
 // transposed, for A^H ubar): the same pairs with the two values exchanged.
-template <int PDE, int DIM, int KIND, bool MIXED, int G, int TPL, bool TRANS = false, bool CHIK = false>
-__global__ __launch_bounds__(kSymBS / TPL) void k_apply_sym(SymArgs A) {
+template <int PDE, int DIM, int KIND, bool MIXED, int G, int TPL, bool TRANS = false, bool CHIK = false, int TS = kSymBS>
+__global__ __launch_bounds__(TS / TPL) void k_apply_sym(SymArgs A) {
     // mixed 3D Helmholtz DL and DL + ch*SL: value and accumulation fused,
     // the products and the 64-term running sums in FP32 (added into FP64
     // after every 32-step pass); in FP64 the fused form's larger LDS record
@@ -210,14 +225,14 @@ __global__ __launch_bounds__(kSymBS / TPL) void k_apply_sym(SymArgs A) {
     constexpr bool FUSEDL = MIXED && PDE == INTI_LAPLACE && DIM == 3;
     using R = std::conditional_t<FUSED, SymRecF<CHIK>, SymRec<PDE, DIM, KIND>>;
     constexpr bool CPLX = PDE == INTI_HELMHOLTZ;
-    constexpr int BS = kSymBS / TPL;  // threads
+    constexpr int BS = TS / TPL;  // threads
     constexpr int NW = BS / 64;       // waves
-    // two waves add their transposed sums onto zero with LDS atomics (two
-    // addends: the result does not depend on their order); more waves write
-    // their own rows, added in wave order
+    // one wave stores its transposed sums itself; two waves add theirs onto
+    // zero with LDS atomics (two addends: the result does not depend on
+    // their order); more waves write their own rows, added in wave order
     constexpr bool RED_ADD = NW == 2;
-    __shared__ double2 s_src[R::NS][kSymBS];
-    __shared__ double2 s_red[RED_ADD ? 1 : NW][kSymBS];
+    __shared__ double2 s_src[R::NS][TS];
+    __shared__ double2 s_red[NW <= 2 ? 1 : NW][NW == 1 ? 1 : TS];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nxt = ((lane + 1) & 63) << 2;  // ds_bpermute address of lane l+1
     const int far = ((lane + 32) & 63) << 2;  // and of lane l+32
@@ -238,7 +253,7 @@ __global__ __launch_bounds__(kSymBS / TPL) void k_apply_sym(SymArgs A) {
 #pragma unroll
         for (int t = 0; t < TPL; ++t) {
             double y[3], nv[3], qr, qi;
-            sym_node<DIM, CPLX>(A, J * kSymBS + tid + t * BS, y, nv, qr, qi);
+            sym_node<DIM, CPLX>(A, J * TS + tid + t * BS, y, nv, qr, qi);
             if constexpr (FUSED) R::put(s_src, tid + t * BS, y, nv, qext32(qr, qi, p));
             else R::put(s_src, tid + t * BS, y, nv, qr, qi);
             if constexpr (RED_ADD) s_red[0][tid + t * BS] = make_double2(0.0, 0.0);
@@ -251,9 +266,9 @@ __global__ __launch_bounds__(kSymBS / TPL) void k_apply_sym(SymArgs A) {
         if constexpr (G == 1) {
 #pragma unroll
             for (int t = 0; t < TPL; ++t)
-                sym_node<DIM, CPLX>(A, a * kSymBS + tid + t * BS, xh[t], nh[t], qhr[t], qhi[t]);
+                sym_node<DIM, CPLX>(A, a * TS + tid + t * BS, xh[t], nh[t], qhr[t], qhi[t]);
         }
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < TS / 64; ++u) {
             // Two independent rotating chains of transposed sums: at step s
             // lane l pairs its targets with source (l + s) mod 64 (chain A,
             // running sum aa) and with source (l + s + 32) mod 64 (chain B,
@@ -277,7 +292,7 @@ __global__ __launch_bounds__(kSymBS / TPL) void k_apply_sym(SymArgs A) {
                         qir[t] = qhr[t];
                         qii[t] = qhi[t];
                     } else {
-                        sym_node<DIM, CPLX>(A, I * kSymBS + tid + t * BS, xi[t], ni[t], qir[t], qii[t]);
+                        sym_node<DIM, CPLX>(A, I * TS + tid + t * BS, xi[t], ni[t], qir[t], qii[t]);
                     }
                 }
                 if (diag && gi == gj) {
@@ -488,7 +503,13 @@ __global__ __launch_bounds__(kSymBS / TPL) void k_apply_sym(SymArgs A) {
             double ajr = aar + lane_next(abr, far);
             double aji = CPLX ? aai + lane_next(abi, far) : 0.0;
             if (trans) {
-                if constexpr (RED_ADD) {
+                if constexpr (NW == 1) {
+                    const int64_t j = J * TS + u * 64 + lane;
+                    if (j < n) {
+                        if constexpr (CPLX) reinterpret_cast<double2 *>(A.part)[a * n + j] = make_double2(ajr, aji);
+                        else A.part[a * n + j] = ajr;
+                    }
+                } else if constexpr (RED_ADD) {
                     double *sr = &s_red[0][u * 64 + lane].x;
                     __hip_atomic_fetch_add(sr, ajr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                     if constexpr (CPLX)
@@ -498,12 +519,12 @@ __global__ __launch_bounds__(kSymBS / TPL) void k_apply_sym(SymArgs A) {
                 }
             }
         }
-        if (trans) {
+        if (NW > 1 && trans) {
             __syncthreads();
 #pragma unroll
             for (int t = 0; t < TPL; ++t) {
                 const int jt = tid + t * BS;
-                const int64_t j = J * kSymBS + jt;
+                const int64_t j = J * TS + jt;
                 if (j < n) {
                     double vr = s_red[0][jt].x, vi = s_red[0][jt].y;
                     if constexpr (!RED_ADD) {
@@ -524,7 +545,7 @@ __global__ __launch_bounds__(kSymBS / TPL) void k_apply_sym(SymArgs A) {
         if (I >= T) continue;
 #pragma unroll
         for (int t = 0; t < TPL; ++t) {
-            const int64_t i = I * kSymBS + tid + t * BS;
+            const int64_t i = I * TS + tid + t * BS;
             if (i >= n) continue;
             const int64_t off = (diag ? a : b) * n + i;
             // in a diagonal block, tile gi > 0 already holds its transposed
@@ -549,78 +570,92 @@ using SymFn = void (*)(const SymArgs &, int64_t, hipStream_t);
 // targets per lane (one LDS read of a source serves TPL pairs): 4 for the
 // cheap Laplace pairs, 2 for 3D Helmholtz, 1 for the 2D Helmholtz kernels,
 // whose Hankel evaluation already fills the register file (measured best)
-template <int PDE, int DIM, int KIND, bool MIXED, int G, bool TRANS = false>
-static void sym_launcher(const SymArgs &a, int64_t nblocks, hipStream_t s) {
-    constexpr int TPL = PDE == INTI_LAPLACE ? 4 : DIM == 2 ? 1 : 2;
+template <int PDE, int DIM>
+constexpr int sym_tpl() { return PDE == INTI_LAPLACE ? 4 : DIM == 2 ? 1 : 2; }
+
+template <int PDE, int DIM, int KIND, bool MIXED, int G, int TPL, bool TRANS, int TS>
+static void sym_launch(const SymArgs &a, int64_t nblocks, hipStream_t s) {
     // the fused mixed combined field with ch = -i k has its own (smaller) record
     constexpr bool CHIK_KERNEL = MIXED && !TRANS && PDE == INTI_HELMHOLTZ && DIM == 3 && KIND == INTI_COMB_SD;
     if constexpr (CHIK_KERNEL) {
         if (a.ch_ik) {
-            hipLaunchKernelGGL((k_apply_sym<PDE, DIM, KIND, MIXED, G, TPL, TRANS, true>), dim3((unsigned)nblocks),
-                               dim3(kSymBS / TPL), 0, s, a);
+            hipLaunchKernelGGL((k_apply_sym<PDE, DIM, KIND, MIXED, G, TPL, TRANS, true, TS>), dim3((unsigned)nblocks),
+                               dim3(TS / TPL), 0, s, a);
             return;
         }
     }
-    hipLaunchKernelGGL((k_apply_sym<PDE, DIM, KIND, MIXED, G, TPL, TRANS>), dim3((unsigned)nblocks),
-                       dim3(kSymBS / TPL), 0, s, a);
+    hipLaunchKernelGGL((k_apply_sym<PDE, DIM, KIND, MIXED, G, TPL, TRANS, false, TS>), dim3((unsigned)nblocks),
+                       dim3(TS / TPL), 0, s, a);
 }
 
-template <int PDE, int DIM, bool MIXED, int G>
+// TILE nodes per tile (SymPlan): 256 in groups of G tiles, or the one-wave
+// blocks of smaller sums, 64 nodes at one target per lane and 128 at two
+template <int PDE, int DIM, int KIND, bool MIXED, int TILE, int G, bool TRANS = false>
+static void sym_launcher(const SymArgs &a, int64_t nblocks, hipStream_t s) {
+    sym_launch<PDE, DIM, KIND, MIXED, G, TILE == kSymBS ? sym_tpl<PDE, DIM>() : TILE / 64, TRANS, TILE>(a, nblocks, s);
+}
+
+template <int PDE, int DIM, bool MIXED, int TILE, int G>
 static SymFn sym_kind(int kind) {
     switch (kind) {
-        case INTI_SL: return sym_launcher<PDE, DIM, INTI_SL, MIXED, G>;
-        case INTI_DL: return sym_launcher<PDE, DIM, INTI_DL, MIXED, G>;
-        case INTI_ADL: return sym_launcher<PDE, DIM, INTI_ADL, MIXED, G>;
-        case INTI_HS: return sym_launcher<PDE, DIM, INTI_HS, MIXED, G>;
-        case INTI_COMB_SD: return sym_launcher<PDE, DIM, INTI_COMB_SD, MIXED, G>;
-        case INTI_COMB_AH: return sym_launcher<PDE, DIM, INTI_COMB_AH, MIXED, G>;
+        case INTI_SL: return sym_launcher<PDE, DIM, INTI_SL, MIXED, TILE, G>;
+        case INTI_DL: return sym_launcher<PDE, DIM, INTI_DL, MIXED, TILE, G>;
+        case INTI_ADL: return sym_launcher<PDE, DIM, INTI_ADL, MIXED, TILE, G>;
+        case INTI_HS: return sym_launcher<PDE, DIM, INTI_HS, MIXED, TILE, G>;
+        case INTI_COMB_SD: return sym_launcher<PDE, DIM, INTI_COMB_SD, MIXED, TILE, G>;
+        case INTI_COMB_AH: return sym_launcher<PDE, DIM, INTI_COMB_AH, MIXED, TILE, G>;
     }
     return nullptr;
 }
 
-// G in {1, 2, 4}
-template <int PDE, int DIM>
-static SymFn sym_pick_pd(int kind, int mixed, int G) {
-    if (mixed) {
-        if (G == 1) return sym_kind<PDE, DIM, true, 1>(kind);
-        if (G == 2) return sym_kind<PDE, DIM, true, 2>(kind);
-        if (G == 4) return sym_kind<PDE, DIM, true, 4>(kind);
-    } else {
-        if (G == 1) return sym_kind<PDE, DIM, false, 1>(kind);
-        if (G == 2) return sym_kind<PDE, DIM, false, 2>(kind);
-        if (G == 4) return sym_kind<PDE, DIM, false, 4>(kind);
-    }
+template <int PDE, int DIM, bool MIXED>
+static SymFn sym_tile(int kind, int tile, int G) {
+    if (tile == 64) return sym_kind<PDE, DIM, MIXED, 64, 1>(kind);
+    if constexpr (!(PDE == INTI_HELMHOLTZ && DIM == 2))
+        if (tile == 128) return sym_kind<PDE, DIM, MIXED, 128, 1>(kind);
+    if (tile != kSymBS) return nullptr;
+    if (G == 1) return sym_kind<PDE, DIM, MIXED, kSymBS, 1>(kind);
+    if (G == 2) return sym_kind<PDE, DIM, MIXED, kSymBS, 2>(kind);
+    if (G == 4) return sym_kind<PDE, DIM, MIXED, kSymBS, 4>(kind);
     return nullptr;
+}
+template <int PDE, int DIM>
+static SymFn sym_pick_pd(int kind, int mixed, int tile, int G) {
+    return mixed ? sym_tile<PDE, DIM, true>(kind, tile, G) : sym_tile<PDE, DIM, false>(kind, tile, G);
 }
 
 // transposed FP64 sums of the kinds with a pullback: SL is its own
 // transpose; DL and c0 SL + c1 DL need the exchanged values
-template <int PDE, int DIM, int G>
+template <int PDE, int DIM, int TILE, int G>
 static SymFn sym_trans_kind(int kind) {
     switch (kind) {
-        case INTI_SL: return sym_launcher<PDE, DIM, INTI_SL, false, G>;
-        case INTI_DL: return sym_launcher<PDE, DIM, INTI_DL, false, G, true>;
-        case INTI_COMB_SD: return sym_launcher<PDE, DIM, INTI_COMB_SD, false, G, true>;
+        case INTI_SL: return sym_launcher<PDE, DIM, INTI_SL, false, TILE, G>;
+        case INTI_DL: return sym_launcher<PDE, DIM, INTI_DL, false, TILE, G, true>;
+        case INTI_COMB_SD: return sym_launcher<PDE, DIM, INTI_COMB_SD, false, TILE, G, true>;
     }
     return nullptr;
 }
 
 template <int PDE, int DIM>
-static SymFn sym_trans_pick_pd(int kind, int G) {
-    if (G == 1) return sym_trans_kind<PDE, DIM, 1>(kind);
-    if (G == 2) return sym_trans_kind<PDE, DIM, 2>(kind);
-    if (G == 4) return sym_trans_kind<PDE, DIM, 4>(kind);
+static SymFn sym_trans_pick_pd(int kind, int tile, int G) {
+    if (tile == 64) return sym_trans_kind<PDE, DIM, 64, 1>(kind);
+    if constexpr (!(PDE == INTI_HELMHOLTZ && DIM == 2))
+        if (tile == 128) return sym_trans_kind<PDE, DIM, 128, 1>(kind);
+    if (tile != kSymBS) return nullptr;
+    if (G == 1) return sym_trans_kind<PDE, DIM, kSymBS, 1>(kind);
+    if (G == 2) return sym_trans_kind<PDE, DIM, kSymBS, 2>(kind);
+    if (G == 4) return sym_trans_kind<PDE, DIM, kSymBS, 4>(kind);
     return nullptr;
 }
 
-SymFn sym_trans_pick_lap2(int kind, int G);
-SymFn sym_trans_pick_lap3(int kind, int G);
-SymFn sym_trans_pick_helm2(int kind, int G);
-SymFn sym_trans_pick_helm3(int kind, int G);
+SymFn sym_trans_pick_lap2(int kind, int tile, int G);
+SymFn sym_trans_pick_lap3(int kind, int tile, int G);
+SymFn sym_trans_pick_helm2(int kind, int tile, int G);
+SymFn sym_trans_pick_helm3(int kind, int tile, int G);
 
-SymFn sym_pick_lap2(int kind, int mixed, int G);
-SymFn sym_pick_lap3(int kind, int mixed, int G);
-SymFn sym_pick_helm2(int kind, int mixed, int G);
-SymFn sym_pick_helm3(int kind, int mixed, int G);
+SymFn sym_pick_lap2(int kind, int mixed, int tile, int G);
+SymFn sym_pick_lap3(int kind, int mixed, int tile, int G);
+SymFn sym_pick_helm2(int kind, int mixed, int tile, int G);
+SymFn sym_pick_helm3(int kind, int mixed, int tile, int G);
 
 }  // namespace inti

@@ -9,22 +9,6 @@
 
 namespace inti {
 
-struct ReduceArgs {
-    int64_t m;
-    int split;
-    const double *part;  // nr x split x m
-    int64_t ldx, ldy;    // leading dimensions of x and y (elements)
-    const int32_t *rowptr;
-    const int32_t *colind;
-    const double *cval;
-    const double *x;  // density (for the correction and identity terms)
-    double *y;
-    double ar, ai, br, bi, cr, ci;
-    double pr, pi;  // post factor of the direct sum
-    int beta_zero;
-    int has_id;
-};
-
 // y_i = alpha * (post * sum_c part[c][i] + (dA x)_i + cid x_i) + beta * y_i,
 // one right-hand side per blockIdx.y
 template <bool CPLX>
@@ -50,48 +34,7 @@ __global__ __launch_bounds__(256) void k_reduce(ReduceArgs a) {
 #pragma unroll 8
         for (int c = 0; c < a.split; ++c) sr += a.part[pbase + (int64_t)c * a.m + i];
     }
-    {
-        const double tr = a.pr * sr - a.pi * si, ti = a.pr * si + a.pi * sr;
-        sr = tr;
-        si = ti;
-    }
-    if (a.rowptr) {
-        const int32_t p0 = a.rowptr[i], p1 = a.rowptr[i + 1];
-        for (int32_t p = p0; p < p1; ++p) {
-            const int32_t j = a.colind[p];
-            if constexpr (CPLX) {
-                const double vr = a.cval[2 * p], vi = a.cval[2 * p + 1];
-                const double xr = x[2 * j], xi = x[2 * j + 1];
-                sr += vr * xr - vi * xi;
-                si += vr * xi + vi * xr;
-            } else {
-                sr += a.cval[p] * x[j];
-            }
-        }
-    }
-    if (a.has_id) {
-        if constexpr (CPLX) {
-            const double xr = x[2 * i], xi = x[2 * i + 1];
-            sr += a.cr * xr - a.ci * xi;
-            si += a.cr * xi + a.ci * xr;
-        } else {
-            sr += a.cr * x[i];
-        }
-    }
-    if constexpr (CPLX) {
-        double yr = a.ar * sr - a.ai * si, yi = a.ar * si + a.ai * sr;
-        if (!a.beta_zero) {
-            const double or_ = y[2 * i], oi = y[2 * i + 1];
-            yr += a.br * or_ - a.bi * oi;
-            yi += a.br * oi + a.bi * or_;
-        }
-        y[2 * i] = yr;
-        y[2 * i + 1] = yi;
-    } else {
-        double yr = a.ar * sr;
-        if (!a.beta_zero) yr += a.br * y[i];
-        y[i] = yr;
-    }
+    reduce_epilogue<CPLX>(a, i, x, y, sr, si);
 }
 
 // Long correction rows (a stencil of many elements per target: hundreds of
@@ -168,11 +111,20 @@ static ApplyFn pick_apply(int pde, int dim, int kind, int mixed, int nr) {
     return nullptr;
 }
 
-static SymFn pick_sym(int pde, int dim, int kind, int mixed, int G) {
-    if (pde == INTI_LAPLACE && dim == 2) return sym_pick_lap2(kind, mixed, G);
-    if (pde == INTI_LAPLACE && dim == 3) return sym_pick_lap3(kind, mixed, G);
-    if (pde == INTI_HELMHOLTZ && dim == 2) return sym_pick_helm2(kind, mixed, G);
-    if (pde == INTI_HELMHOLTZ && dim == 3) return sym_pick_helm3(kind, mixed, G);
+static RowFn pick_row(int pde, int dim, int kind, int mixed) {
+    if (pde == INTI_LAPLACE && dim == 2) return row_pick_lap2(kind, mixed);
+    if (pde == INTI_LAPLACE && dim == 3) return row_pick_lap3(kind, mixed);
+    if (pde == INTI_HELMHOLTZ && dim == 2) return row_pick_helm2(kind, mixed);
+    if (pde == INTI_HELMHOLTZ && dim == 3) return row_pick_helm3(kind, mixed);
+    if (pde == kHelmCK && dim == 3 && !mixed) return row_pick_helm3c(kind);
+    return nullptr;
+}
+
+static SymFn pick_sym(int pde, int dim, int kind, int mixed, const SymPlan &P) {
+    if (pde == INTI_LAPLACE && dim == 2) return sym_pick_lap2(kind, mixed, P.tile, P.G);
+    if (pde == INTI_LAPLACE && dim == 3) return sym_pick_lap3(kind, mixed, P.tile, P.G);
+    if (pde == INTI_HELMHOLTZ && dim == 2) return sym_pick_helm2(kind, mixed, P.tile, P.G);
+    if (pde == INTI_HELMHOLTZ && dim == 3) return sym_pick_helm3(kind, mixed, P.tile, P.G);
     return nullptr;
 }
 
@@ -183,28 +135,82 @@ int op_kernel_pde(const Op *op) { return op->pde == INTI_HELMHOLTZ && op->kimag 
 // plain direct sum runs
 constexpr size_t kSymMaxBytes = size_t(4) << 30;
 
-// Symmetric plan for one right-hand side of op: tiles of 256 in groups of G
-// (the smallest of 1, 2, 4 whose S x n partials fit kSymMaxBytes). False if
-// the operator does not qualify.
-static bool plan_sym(const Op *op, int kind, int nr, int &G, int64_t &T, int64_t &S) {
-    if (op->sym == 0 || nr != 1 || op->trg != op->src || kind >= INTI_FF_SL || op->kimag != 0.0) return false;
+// Partial sums of the small-tile plans (n^2 / tile of them): the gain of the
+// small tiles is not worth more memory than this.
+constexpr size_t kSymSmallBytes = size_t(512) << 20;
+
+// Tiles of 256 nodes keep the partial sums few, but a sum of n nodes is then
+// only T (T + 1) / 2 blocks, and with a few waves per SIMD the chip waits on
+// its dependency chains and on the last round of blocks. Smaller sums are
+// therefore cut into one-wave blocks of 64 nodes (one target per lane, below
+// 12 waves per CU of 128-node blocks, about 10,000 nodes) or 128 nodes (two
+// targets per lane, below 72 tile pairs of 256 nodes per CU, about 49,000).
+// The 2D Helmholtz pairs take 64 wherever the partial sums allow: their
+// Hankel evaluation branches on the argument, and one wave without barriers
+// waits for no other wave's branch. Measured, us per apply with 256 / 128 /
+// 64-node tiles (before: one direction below 8,200 nodes):
+//   3D Helmholtz CF FP64   4,320: 101 / 57 / 44 (one direction 83)
+//                         12,000: 253 / 213 / 206    24,000: 837 / 734 / 750
+//                         40,000: 2001 / 1926 / 2084 63,480: 4826 / 4894 / 5320
+//   3D Laplace SL FP64     4,320: 55 / 22 / 19 (29)  8,500: 58 / 42 / 41
+//                         24,000: 214 / 188 / 216    63,480: 1125 / 1171 / 1463
+//   2D Helmholtz CF FP64   6,006: 479 / 437 / 251 (500)  30,720: 4222 / 4114 / 3869
+//   2D Helmholtz CF mixed  6,006: 123 / 120 / 82 (146)   40,000: 2011 / 2032 / 1999
+// Sums of 256 nodes or fewer run in one direction (k_apply_row). An explicit
+// group keeps tiles of 256. Beyond kSymMaxBytes of partial sums the groups of
+// 2 and 4 tiles halve and quarter them.
+bool plan_sym(const Op *op, int kind, SymPlan &P) {
+    if (op->sym == 0 || op->trg != op->src || kind >= INTI_FF_SL || op->kimag != 0.0) return false;
     const int64_t n = op->src->n;
-    T = (n + kSymBS - 1) / kSymBS;
-    if (T < 2) return false;
-    // automatic mode: only where the triangle of tile pairs fills the GPU
-    // (two blocks per CU); below that the plain sum, whose source range is
-    // split across blocks, is faster
-    if (op->sym == 1 && T * (T + 1) / 2 < 2LL * op->ctx->num_cu) return false;
-    const size_t cw = op_is_complex(op) ? 2 : 1;
+    auto tiles = [n](int tile) { return (n + tile - 1) / tile; };
+    if (tiles(kSymBS) < 2) return false;
+    const size_t es = sizeof(double) * (op_is_complex(op) ? 2 : 1);
+    if (op->sym_group == 0) {
+        const int64_t t128 = tiles(128), t256 = tiles(kSymBS), cu = op->ctx->num_cu;
+        const bool helm2 = op->pde == INTI_HELMHOLTZ && op->dim == 2;
+        int tile = kSymBS;
+        if (helm2 || t128 * (t128 + 1) / 2 < 12 * cu) tile = 64;
+        else if (t256 * (t256 + 1) / 2 < 72 * cu) tile = 128;
+        if (tile < kSymBS && (size_t)tiles(tile) * (size_t)n * es <= kSymSmallBytes) {
+            P = SymPlan{tile, 1, tiles(tile), tiles(tile)};
+            return true;
+        }
+    }
     for (int g : {1, 2, 4}) {
         if (op->sym_group && g != op->sym_group) continue;
-        S = (T + g - 1) / g;
-        if ((size_t)S * (size_t)n * cw * sizeof(double) <= kSymMaxBytes) {
-            G = g;
+        const int64_t T = tiles(kSymBS), S = (T + g - 1) / g;
+        if ((size_t)S * (size_t)n * es <= kSymMaxBytes) {
+            P = SymPlan{kSymBS, g, T, S};
             return true;
         }
     }
     return false;
+}
+
+// Targets per block of the one-launch sum (k_apply_row) for a single
+// right-hand side of m targets and n sources, 0 where another sum is taken.
+// Four targets per block and 64 threads per target keep every thread's
+// source chain short; it reads each source's data once per 16 threads instead
+// of staging it, so it pays where launches, barriers and an idle chip cost
+// more than the loads: few pairs. Against the symmetric sum it is faster up
+// to about 1,800 nodes (3D Helmholtz CF 1,280: 15 / 20 us, 3,000: 41 / 33;
+// 3D Laplace SL 1,280: 8 / 11, 3,000: 23 / 15) and, for 2D Helmholtz, up to
+// 3,400 (CF 3,000: 96 / 150; 4,320: 205 / 171); against the one-direction sum
+// with its second kernel up to 2,400 (Laplace 2,000: 11 / 20; 3,000: 23 / 21)
+// and 3,800 nodes (3D Helmholtz CF 3,000: 40 / 59; 4,320: 85 / 83). The 2D
+// Helmholtz kernels keep it at any size once 4 m threads per CU are in
+// flight: a wave of 4 targets x 16 neighbouring sources takes the same side
+// of the Hankel functions' branch more often than one of 64 targets (CF FP64
+// 12,000: 1264 / 1337 us, 30,720: 7785 / 8235). The chain of a thread is
+// bounded (n <= 8,192) where the targets alone do not fill the chip.
+static int plan_row(const Op *op, int64_t m, int64_t n, bool sym) {
+    if (op->split > 0 || n <= 0) return 0;
+    if (sym && op->sym == 2) return 0;
+    const double pairs = (double)m * (double)n;
+    const bool lap = op->pde == INTI_LAPLACE, helm2 = op->pde == INTI_HELMHOLTZ && op->dim == 2;
+    if (helm2 && !sym && m >= 4LL * op->ctx->num_cu) return 4;
+    const double lim = sym ? (helm2 ? 3400.0 : 1800.0) : (helm2 ? 3400.0 : lap ? 2400.0 : 3800.0);
+    return n <= 8192 && pairs <= lim * lim ? 4 : 0;
 }
 
 KParams op_params(const Op *op, int *eff_kind) {
@@ -286,23 +292,29 @@ static void plan_split(const Op *op, int64_t m, int64_t n, ApplyFn fn, int nr, i
     if (split < 1) split = 1;
 }
 
+// scratch of the column blocks (16, 4, 1) a call of nrhs columns uses
 int apply_reserve(const Op *op, int nrhs) {
     const int cw = op_is_complex(op) ? 2 : 1;
     const int64_t m = op->trg->n, n = op->src->n;
-    int kind = op->kind, G;
-    int64_t T, S;
+    int kind = op->kind;
+    SymPlan sp;
     (void)op_params(op, &kind);
-    // the largest partial buffer of the column blocks (16, 4, 1) a call uses
     size_t bytes = 0;
     for (int nr : {16, 4, 1}) {
-        if (nrhs < nr && nr != 1) continue;
+        if (nrhs < nr) continue;
+        if (nr == 1) {
+            const bool sym = plan_sym(op, kind, sp);
+            if (plan_row(op, m, n, sym)) continue;
+            if (sym) {
+                bytes = std::max(bytes, sizeof(double) * cw * (size_t)sp.S * (size_t)n);
+                continue;
+            }
+        }
         int split;
         int64_t chunk;
         plan_split(op, m, n, pick_apply(op_kernel_pde(op), op->dim, kind, op->precision == INTI_MIXED, nr), nr, split, chunk);
         bytes = std::max(bytes, sizeof(double) * cw * (size_t)m * split * nr);
     }
-    if (nrhs >= 1 && plan_sym(op, kind, 1, G, T, S))
-        bytes = std::max(bytes, sizeof(double) * cw * (size_t)S * (size_t)n);
     void *scr = nullptr;
     return ctx_scratch(op->ctx, kScrPartial, bytes, &scr);
 }
@@ -317,32 +329,40 @@ int launch_apply(const DirectLaunch &L) {
     int kind = op->kind;
     const KParams kp = op_params(op, &kind);
     const bool given = L.part != nullptr;
-    void *scr = nullptr;
     double *part = L.part;
     if (!given) {
         int st = apply_reserve(op, L.nrhs);
         if (st) return st;
+        void *scr = nullptr;
         st = ctx_scratch(ctx, kScrPartial, 0, &scr);
         if (st) return st;
         part = (double *)scr;
     }
-    int st = INTI_OK;
     const int64_t ntiles = (m + kApplyBS - 1) / kApplyBS;
-    int symG = 0;
-    int64_t symT = 0, symS = 0;
-    const bool sym = !given && plan_sym(op, kind, 1, symG, symT, symS);
-    if (sym) {
-        const size_t bytes = sizeof(double) * cw * (size_t)symS * (size_t)n;
-        st = ctx_scratch(ctx, kScrPartial, bytes, &scr);
-        if (st) return st;
-        part = (double *)scr;
-    }
+    SymPlan sp{};
+    const bool sym = !given && plan_sym(op, kind, sp);
     for (int r0 = 0; r0 < L.nrhs;) {
         const int left = L.nrhs - r0;
         const int nr = left >= 16 ? 16 : left >= 4 ? 4 : 1;
         const double *xr = L.x + (int64_t)r0 * L.ldx * cw;
         double *yr = L.y + (int64_t)r0 * L.ldy * cw;
-        ApplyFn fn = sym && nr == 1 ? nullptr : pick_apply(op_kernel_pde(op), op->dim, kind, op->precision == INTI_MIXED, nr);
+        ReduceArgs ra;
+        ra.m = m;
+        ra.ldx = L.ldx; ra.ldy = L.ldy;
+        const int cl = csr_lanes(op->corr);
+        ra.rowptr = op->corr && !cl ? op->corr->rowptr : nullptr;
+        ra.colind = op->corr && !cl ? op->corr->colind : nullptr;
+        ra.cval = op->corr && !cl ? op->corr->val : nullptr;
+        ra.x = xr; ra.y = yr;
+        ra.ar = L.alpha[0]; ra.ai = L.alpha[1];
+        ra.br = L.beta[0]; ra.bi = L.beta[1];
+        ra.beta_zero = (L.beta[0] == 0.0 && L.beta[1] == 0.0);
+        ra.cr = op->cid[0]; ra.ci = op->cid[1];
+        ra.pr = kp.postr; ra.pi = kp.posti;
+        ra.has_id = (op->cid[0] != 0.0 || op->cid[1] != 0.0);
+        const int tb = nr == 1 ? plan_row(op, m, n, sym) : 0;
+        RowFn rfn = tb ? pick_row(op_kernel_pde(op), op->dim, kind, op->precision == INTI_MIXED) : nullptr;
+        ApplyFn fn = rfn || (sym && nr == 1) ? nullptr : pick_apply(op_kernel_pde(op), op->dim, kind, op->precision == INTI_MIXED, nr);
         int split = 1;
         int64_t chunk = n;
         if (fn) plan_split(op, m, n, fn, nr, split, chunk);
@@ -353,21 +373,35 @@ int launch_apply(const DirectLaunch &L) {
             const int64_t cap = (int64_t)(L.part_bytes / per);
             if (cap < 1)
                 return set_error(ctx, INTI_ERR_SIZE, "apply: the partial sums of this shape exceed the buffer");
-            if (split > cap) {
+            if (fn && split > cap) {
                 const int64_t stiles = (n + kApplyBS - 1) / kApplyBS;
                 chunk = (stiles + cap - 1) / cap * kApplyBS;
                 split = (int)((n + chunk - 1) / chunk);
             }
         }
         int nsplit = split;
-        if (n > 0 && nr == 1 && sym) {
-            SymFn sfn = pick_sym(op->pde, op->dim, kind, op->precision == INTI_MIXED, symG);
+        if (rfn) {
+            RowArgs a;
+            a.s.m = m; a.s.n = n;
+            a.s.tstride = m; a.s.sstride = n;
+            a.s.tx = op->trg->coords; a.s.tn = op->trg->normals;
+            a.s.sx = op->src->coords; a.s.sn = op->src->normals; a.s.sw = op->src->weights;
+            a.s.x = xr; a.s.ldx = L.ldx; a.s.part = nullptr; a.s.split = 0; a.s.chunk = 0;
+            a.s.p = kp;
+            a.e = ra;
+            a.tb = tb;
+            if (ctx->profiling) INTI_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
+            rfn(a, dim3((unsigned)((m + tb - 1) / tb)), ctx->stream);
+            INTI_HIP(ctx, hipGetLastError());
+            if (ctx->profiling) INTI_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
+        } else if (n > 0 && nr == 1 && sym) {
+            SymFn sfn = pick_sym(op->pde, op->dim, kind, op->precision == INTI_MIXED, sp);
             if (!sfn) return set_error(ctx, INTI_ERR_UNSUPPORTED, "no symmetric kernel for this operator");
             SymArgs a;
             a.n = n;
             a.xy = op->src->coords; a.nrm = op->src->normals; a.w = op->src->weights;
             a.x = xr; a.part = part;
-            a.ntiles = symT; a.ngroups = symS;
+            a.ntiles = sp.T; a.ngroups = sp.S;
             a.distinct = op->src->distinct ? 1 : 0;
             // c0 SL + c1 DL with c0 = -i k c1 (the combined field of the
             // reference's examples): ch q needs no LDS slot of its own
@@ -377,10 +411,10 @@ int launch_apply(const DirectLaunch &L) {
                           : 0;
             a.p = kp;
             if (ctx->profiling) INTI_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
-            sfn(a, symS * (symS + 1) / 2, ctx->stream);
+            sfn(a, sp.S * (sp.S + 1) / 2, ctx->stream);
             INTI_HIP(ctx, hipGetLastError());
             if (ctx->profiling) INTI_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
-            nsplit = (int)symS;
+            nsplit = (int)sp.S;
         } else if (n > 0) {
             if (!fn) return set_error(ctx, INTI_ERR_UNSUPPORTED, "no direct-sum kernel for this operator");
             ApplyArgs a;
@@ -396,24 +430,14 @@ int launch_apply(const DirectLaunch &L) {
             INTI_HIP(ctx, hipGetLastError());
             if (ctx->profiling) INTI_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
         }
-        ReduceArgs ra;
-        ra.m = m; ra.split = n > 0 ? nsplit : 0; ra.part = part;
-        ra.ldx = L.ldx; ra.ldy = L.ldy;
-        const int cl = csr_lanes(op->corr);
-        ra.rowptr = op->corr && !cl ? op->corr->rowptr : nullptr;
-        ra.colind = op->corr && !cl ? op->corr->colind : nullptr;
-        ra.cval = op->corr && !cl ? op->corr->val : nullptr;
-        ra.x = xr; ra.y = yr;
-        ra.ar = L.alpha[0]; ra.ai = L.alpha[1];
-        ra.br = L.beta[0]; ra.bi = L.beta[1];
-        ra.beta_zero = (L.beta[0] == 0.0 && L.beta[1] == 0.0);
-        ra.cr = op->cid[0]; ra.ci = op->cid[1];
-        ra.pr = kp.postr; ra.pi = kp.posti;
-        ra.has_id = (op->cid[0] != 0.0 || op->cid[1] != 0.0);
-        dim3 rg((unsigned)((m + 255) / 256), (unsigned)nr);
-        if (cplx) hipLaunchKernelGGL(k_reduce<true>, rg, dim3(256), 0, ctx->stream, ra);
-        else hipLaunchKernelGGL(k_reduce<false>, rg, dim3(256), 0, ctx->stream, ra);
-        INTI_HIP(ctx, hipGetLastError());
+        if (!rfn) {
+            ra.split = n > 0 ? nsplit : 0;
+            ra.part = part;
+            dim3 rg((unsigned)((m + 255) / 256), (unsigned)nr);
+            if (cplx) hipLaunchKernelGGL(k_reduce<true>, rg, dim3(256), 0, ctx->stream, ra);
+            else hipLaunchKernelGGL(k_reduce<false>, rg, dim3(256), 0, ctx->stream, ra);
+            INTI_HIP(ctx, hipGetLastError());
+        }
         if (cl) {
             CsrAddArgs ca;
             ca.m = m; ca.ldx = L.ldx; ca.ldy = L.ldy;

@@ -176,8 +176,8 @@ class IntegralOperator:
 
     def set_symmetric(self, mode, group=0):
         """Symmetric evaluation when target is source (single right-hand
-        side): mode 0 off, 1 automatic (default: where the work fills the
-        GPU), 2 wherever it applies; group = tiles of 256 nodes per work group
+        side): mode 0 off, 1 automatic (default: where it is the faster
+        sum), 2 wherever it applies; group = tiles of 256 nodes per work group
         (0 automatic)."""
         self.ctx.check(self.ctx.lib.inti_op_set_symmetric(self.handle, int(mode), int(group)))
 

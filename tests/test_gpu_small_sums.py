@@ -1,0 +1,99 @@
+"""The one-launch sum of few targets and the symmetric sum with 64- and
+128-node tiles, at the edges of their ranges and of their tiles: against the
+oracle (FP64 <= 1e-12, the bar of every direct sum; mixed <= 1e-6) on all rows
+of the small sizes and on the first and last rows of the large ones. The
+densities are random, the nodes a spiral on the sphere or an ellipse."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print(*a, flush=True)
+
+
+def _nodes(inti, dim, n, seed=0):
+    i = np.arange(n) + 0.5
+    if dim == 3:
+        pol, az = np.arccos(1 - 2 * i / n), np.pi * (1 + 5 ** 0.5) * i
+        X = np.stack([np.cos(az) * np.sin(pol), np.sin(az) * np.sin(pol), np.cos(pol)])
+    else:
+        X = np.stack([np.cos(2 * np.pi * i / n), 0.6 * np.sin(2 * np.pi * i / n)])
+    N = X / np.linalg.norm(X, axis=0)
+    w = np.random.default_rng(seed).uniform(0.5, 1.5, n) / n
+    return inti.Quadrature(X, N, w, np.zeros((1, 0), dtype=np.int64))
+
+
+def _kernel(inti, pde, dim, kind):
+    op = inti.Laplace(dim=dim) if pde == 0 else inti.Helmholtz(k=7.3, dim=dim)
+    if kind == 4:
+        c = (-7.3j, 1.0) if pde else (0.4, 1.0)
+        return inti.CombinedFieldKernel(op, *c, "SD"), c
+    names = {0: inti.SingleLayerKernel, 1: inti.DoubleLayerKernel, 2: inti.AdjointDoubleLayerKernel,
+             3: inti.HyperSingularKernel}
+    return names[kind](op), None
+
+
+def _check(inti, oracle, pde, dim, kind, Q, T, precision, alpha=1.0, beta=0.0, identity=0.0):
+    k = 7.3 if pde else 0.0
+    K, coefs = _kernel(inti, pde, dim, kind)
+    A = inti.IntegralOperator(K, T, Q, precision=precision)
+    rng = np.random.default_rng(3)
+    n, m = len(Q), len(T)
+    x = rng.normal(size=n) + (1j * rng.normal(size=n) if pde else 0.0)
+    y0 = rng.normal(size=m) + (1j * rng.normal(size=m) if pde else 0.0)
+    if identity:
+        A.set_identity(identity)
+    y = A.apply(x, y0.copy(), alpha=alpha, beta=beta)  # writes into its y
+    ref = np.zeros(m, dtype=np.complex128)
+    blocks = [(0, m)] if m * n <= 1.7e7 else [(0, 130), (m - 130, m)]
+    rows = np.concatenate([np.arange(*b) for b in blocks])
+    for b in blocks:
+        r = oracle.matvec(pde, dim, kind, k, T, Q, x, coefs=coefs, rows=b)
+        ref[b[0]:b[1]] = r[b[0]:b[1]]
+    ref = alpha * (ref + (identity * x if identity else 0.0)) + beta * y0
+    err, size = np.linalg.norm((y - ref)[rows]), np.linalg.norm(ref[rows])
+    say(f"[gpu] pde {pde} dim {dim} kind {kind} {precision} m={m} n={n}: {err:.2e} of {size:.2e}")
+    assert err <= (1e-12 if precision == "fp64" else 1e-6) * size  # (one node alone: both are zero)
+
+
+@pytest.mark.parametrize("pde,dim,kind", [(0, 2, 1), (0, 3, 0), (0, 3, 3), (1, 2, 4), (1, 3, 4), (1, 3, 2)])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("n", [1, 3, 65, 257, 1799, 1801, 3401])
+def test_square(inti, oracle, pde, dim, kind, precision, n):
+    Q = _nodes(inti, dim, n)
+    _check(inti, oracle, pde, dim, kind, Q, Q, precision)
+
+
+# the 64 / 128 and 128 / 256 tile edges (two partial tiles among them)
+@pytest.mark.parametrize("pde,dim,kind,n", [(0, 3, 1, 9855), (0, 3, 1, 9985), (1, 3, 4, 9857), (1, 3, 4, 10050),
+                                            (0, 2, 0, 48705), (0, 3, 0, 49025), (1, 3, 4, 48897), (1, 2, 4, 46000)])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_tile_edges(inti, oracle, pde, dim, kind, n, precision):
+    Q = _nodes(inti, dim, n)
+    _check(inti, oracle, pde, dim, kind, Q, Q, precision)
+
+
+# targets that are not the sources: few and many, with alpha, beta
+@pytest.mark.parametrize("pde,dim,kind", [(0, 3, 1), (1, 2, 0), (1, 3, 4)])
+@pytest.mark.parametrize("m,n", [(1, 5000), (5, 8192), (7, 8193), (1023, 700), (1025, 9000), (2501, 640)])
+def test_rectangular(inti, oracle, pde, dim, kind, m, n):
+    Q = _nodes(inti, dim, n)
+    T = _nodes(inti, dim, m, seed=1)
+    T = inti.Quadrature(1.7 * T.coords, T.normals, T.weights, T.qtags)
+    _check(inti, oracle, pde, dim, kind, Q, T, "fp64", alpha=1.3, beta=-0.4)
+
+
+@pytest.mark.parametrize("n", [500, 5000])
+def test_identity(inti, oracle, n):
+    Q = _nodes(inti, 3, n)
+    _check(inti, oracle, 1, 3, 4, Q, Q, "fp64", alpha=0.5 - 0.2j, beta=0.3j, identity=0.5 + 0.1j)
+
+
+@pytest.mark.parametrize("n", [700, 1500, 9000, 20000])
+def test_repeat_is_bit_identical(inti, n):
+    Q = _nodes(inti, 3, n)
+    A = inti.IntegralOperator(_kernel(inti, 1, 3, 4)[0], Q, Q)
+    x = np.random.default_rng(5).normal(size=n) + 0j
+    assert np.array_equal(A @ x, A @ x)
