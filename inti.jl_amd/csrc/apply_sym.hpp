@@ -221,8 +221,10 @@ __global__ __launch_bounds__(TS / TPL) void k_apply_sym(SymArgs A) {
     // mixed 3D Laplace (every kind): 1/d from the FP32 unit,
     // the values, their products and the 64-term running sums in FP32, added
     // into FP64 after every pass, as above (the distance and the normal dot
-    // products stay FP64)
-    constexpr bool FUSEDL = MIXED && PDE == INTI_LAPLACE && DIM == 3;
+    // products stay FP64). The 64-node tiles keep FP64 products and sums:
+    // their sizes were always summed so, and the FP32 ones would cost
+    // accuracy there (SL, 5,880 nodes: 8e-9 against 5e-8)
+    constexpr bool FUSEDL = MIXED && PDE == INTI_LAPLACE && DIM == 3 && TS > 64;
     using R = std::conditional_t<FUSED, SymRecF<CHIK>, SymRec<PDE, DIM, KIND>>;
     constexpr bool CPLX = PDE == INTI_HELMHOLTZ;
     constexpr int BS = TS / TPL;  // threads
