@@ -48,8 +48,9 @@ struct Quad {
     double *weights = nullptr;  // n
     double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};  // bounding box
     // no two nodes within 2x the coincidence tolerance: pairs of different
-    // nodes then never need the coincident-point mask
-    bool distinct = false;
+    // nodes then never need the coincident-point mask (decided when the first
+    // operator with this quadrature as target and source is created)
+    mutable bool distinct = false, distinct_known = false;
 };
 
 // CSR with 0-based int32 indices; values real (double) or complex

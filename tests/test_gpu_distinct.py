@@ -1,0 +1,38 @@
+"""Coincident nodes of a quadrature, found when its first operator is made:
+a node repeated within a tile of 256, in the next tile or in the last,
+partial one, a pair closer than the coincidence tolerance apart, and none.
+The symmetric sum drops its coincidence mask only for distinct nodes; with a
+coincident pair left unmasked the sums are infinite or NaN, so the apply is
+compared with the oracle (FP64 <= 1e-12)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("shuffled", [False, True])
+@pytest.mark.parametrize("pair", [None, (10, 200), (255, 256), (3, 2299), (700, 1900)])
+@pytest.mark.parametrize("gap", [0.0, 4e-15])
+def test_coincident_nodes(inti, oracle, dim, shuffled, pair, gap):
+    n = 2300
+    i = np.arange(n) + 0.5
+    if dim == 3:
+        pol, az = np.arccos(1 - 2 * i / n), np.pi * (1 + 5 ** 0.5) * i
+        X = np.stack([np.cos(az) * np.sin(pol), np.sin(az) * np.sin(pol), np.cos(pol)])
+    else:
+        X = np.stack([np.cos(2 * np.pi * i / n), np.sin(2 * np.pi * i / n)])
+    rng = np.random.default_rng(0)
+    if shuffled:
+        X = X[:, rng.permutation(n)]
+    if pair:
+        X[:, pair[1]] = X[:, pair[0]]
+        X[0, pair[1]] += gap
+    Q = inti.Quadrature(X, X / np.linalg.norm(X, axis=0), np.full(n, 1.0 / n), np.zeros((1, 0), dtype=np.int64))
+    A = inti.IntegralOperator(inti.SingleLayerKernel(inti.Laplace(dim=dim)), Q, Q)
+    A.set_symmetric(2)
+    x = rng.normal(size=n)
+    y, ref = A @ x, oracle.matvec(0, dim, 0, 0.0, Q, Q, x).real
+    print(f"[gpu] dim {dim} shuffled {shuffled} pair {pair} gap {gap}: "
+          f"{np.linalg.norm(y - ref) / np.linalg.norm(ref):.2e}", flush=True)
+    assert np.linalg.norm(y - ref) <= 1e-12 * np.linalg.norm(ref)
