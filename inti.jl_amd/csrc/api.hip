@@ -873,18 +873,15 @@ int inti_lsq_build_types(inti_ctx *ctx, int is_complex, int nrows, int ntypes, c
 }
 
 // ----------------------------------------------------------------- solvers
-// host pointers: stage b and x on the device for the solve
+// host pointers: stage b and x on the device for the solve, in the context's
+// staging buffers (the solvers themselves use none of them)
 struct Staged {
     void *b = nullptr, *x = nullptr;
-    ~Staged() {
-        if (b) (void)hipFree(b);
-        if (x) (void)hipFree(x);
-    }
 };
 
 static int stage_in(Ctx *ctx, Staged &S, size_t bytes, const double *b, const double *x) {
-    if (hipMalloc(&S.b, bytes) != hipSuccess || hipMalloc(&S.x, bytes) != hipSuccess)
-        return set_error(ctx, INTI_ERR_NOMEM, "solve: allocation failed");
+    if (int st = ctx_scratch(ctx, kScrX, bytes, &S.b)) return st;
+    if (int st = ctx_scratch(ctx, kScrY, bytes, &S.x)) return st;
     INTI_HIP(ctx, hipMemcpyAsync(S.b, b, bytes, hipMemcpyHostToDevice, ctx->stream));
     INTI_HIP(ctx, hipMemcpyAsync(S.x, x, bytes, hipMemcpyHostToDevice, ctx->stream));
     return INTI_OK;
