@@ -811,21 +811,6 @@ SymAdjFn pick_sym(int kind) {
 // passes run
 constexpr size_t kAdjSymMaxBytes = size_t(4) << 30;
 
-struct Dev {
-    void *p = nullptr;
-    hipStream_t s = nullptr;
-    ~Dev() {
-        if (p) {
-            (void)hipStreamSynchronize(s);
-            (void)hipFree(p);
-        }
-    }
-    bool alloc(hipStream_t st, size_t bytes) {
-        s = st;
-        return hipMalloc(&p, bytes ? bytes : 8) == hipSuccess;
-    }
-};
-
 // chunks of the inner index so that the grid has several blocks per CU
 void plan(int64_t own, int64_t inner, int num_cu, int &split, int64_t &chunk) {
     const int64_t tiles = (own + kAdjBS - 1) / kAdjBS;
@@ -931,20 +916,25 @@ static int adjoint_sigma_only(Op *op, const double *ubar, double *sigma_bar) {
     for (int64_t i = 0; i < m; ++i) hc[i] = cplx ? make_double2(ubar[2 * i], -ubar[2 * i + 1]) : make_double2(ubar[i], 0.0);
     std::vector<double> hx;
     if (!cplx) hx.assign(ubar, ubar + m);
-    Dev dc, dx, dpart, dsb;
-    if (!dc.alloc(s, sizeof(double2) * m) || (!cplx && !dx.alloc(s, sizeof(double) * m)) ||
-        !dpart.alloc(s, sizeof(double) * cw * (size_t)S * (size_t)n) || !dsb.alloc(s, sizeof(double) * cw * n))
-        return set_error(ctx, INTI_ERR_NOMEM, "adjoint: allocation failed");
-    INTI_HIP(ctx, hipMemcpyAsync(dc.p, hc.data(), sizeof(double2) * m, hipMemcpyHostToDevice, s));
-    if (!cplx) INTI_HIP(ctx, hipMemcpyAsync(dx.p, hx.data(), sizeof(double) * m, hipMemcpyHostToDevice, s));
-    const double *xc = cplx ? (const double *)dc.p : (const double *)dx.p;  // c, unweighted
+    if (int rc = op_transpose_correction(op)) return rc;
+    double2 *dc;
+    double *dx, *dpart, *dsb;
+    Arena mem(ctx);
+    mem.add(&dc, sizeof(double2) * m);
+    mem.add(&dx, cplx ? 0 : sizeof(double) * m);
+    mem.add(&dpart, sizeof(double) * cw * (size_t)S * (size_t)n);
+    mem.add(&dsb, sizeof(double) * cw * n);
+    if (int rc = mem.commit()) return rc;
+    INTI_HIP(ctx, hipMemcpyAsync(dc, hc.data(), sizeof(double2) * m, hipMemcpyHostToDevice, s));
+    if (!cplx) INTI_HIP(ctx, hipMemcpyAsync(dx, hx.data(), sizeof(double) * m, hipMemcpyHostToDevice, s));
+    const double *xc = cplx ? (const double *)dc : dx;  // c, unweighted
     if (ctx->profiling) INTI_HIP(ctx, hipEventRecord(ctx->ev0, s));
     if (fsym) {
         SymArgs a;
         a.n = n;
         a.xy = op->src->coords; a.nrm = op->src->normals; a.w = nullptr;
         a.x = xc;
-        a.part = (double *)dpart.p;
+        a.part = dpart;
         a.ntiles = sp.T; a.ngroups = S;
         a.distinct = op->src->distinct ? 1 : 0;
         a.ch_ik = 0;  // the transposed sums are FP64 (no staged ch q)
@@ -957,22 +947,22 @@ static int adjoint_sigma_only(Op *op, const double *ubar, double *sigma_bar) {
         a.tx = op->src->coords; a.tn = op->src->normals;
         a.sx = op->trg->coords; a.sn = op->trg->normals; a.sw = nullptr;
         a.x = xc; a.ldx = m;
-        a.part = (double *)dpart.p; a.split = split; a.chunk = chunk;
+        a.part = dpart; a.split = split; a.chunk = chunk;
         a.p = kp;
         fone(&a, dim3((unsigned)(ntiles * split)), s);
     }
     INTI_HIP(ctx, hipGetLastError());
     if (ctx->profiling) INTI_HIP(ctx, hipEventRecord(ctx->ev1, s));
     hipLaunchKernelGGL(k_adj_trans_reduce, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, S, cplx,
-                       (const double *)dpart.p, kp.postr, kp.posti, op->src->weights, (double *)dsb.p);
+                       dpart, kp.postr, kp.posti, op->src->weights, dsb);
     INTI_HIP(ctx, hipGetLastError());
     if (op->corr) {
         hipLaunchKernelGGL(k_adj_corr, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, op->corr_tptr,
-                           op->corr_trow, op->corr_tperm, op->corr->val, cplx, (const double2 *)dc.p,
-                           (double *)dsb.p);
+                           op->corr_trow, op->corr_tperm, op->corr->val, cplx, dc,
+                           dsb);
         INTI_HIP(ctx, hipGetLastError());
     }
-    INTI_HIP(ctx, hipMemcpyAsync(sigma_bar, dsb.p, sizeof(double) * cw * n, hipMemcpyDeviceToHost, s));
+    INTI_HIP(ctx, hipMemcpyAsync(sigma_bar, dsb, sizeof(double) * cw * n, hipMemcpyDeviceToHost, s));
     INTI_HIP(ctx, hipStreamSynchronize(s));
     if (m == n) adjoint_identity(op, cplx, n, ubar, sigma_bar);
     return INTI_OK;
@@ -1060,39 +1050,48 @@ int op_adjoint(Op *op, const double *ubar, const double *sigma, double *sigma_ba
     if (xbar) plan(m, n, ctx->num_cu, split_t, chunk_t);
     const int NVs = 3 + 2 * dim;
     const int64_t nsb = fsym ? symB : (n + 255) / 256;  // kbar partial sums
-    Dev dc, dsg, dpart, dsb, dyb, dnb, dwb, dkp, dxb;
     const size_t part_bytes = fsym ? sizeof(double) * (size_t)symT * NRs * (size_t)n
                                    : std::max(sizeof(double2) * (size_t)split_s * n * NVs,
                                               xbar ? sizeof(double2) * (size_t)split_t * m * dim : 0);
-    if (!dc.alloc(s, sizeof(double2) * m) || !dsg.alloc(s, sizeof(double2) * n) || !dpart.alloc(s, part_bytes) ||
-        !dsb.alloc(s, sizeof(double) * (cplx ? 2 : 1) * n) || !dyb.alloc(s, sizeof(double) * dim * n) ||
-        !dnb.alloc(s, sizeof(double) * dim * n) || !dwb.alloc(s, sizeof(double) * n) ||
-        !dkp.alloc(s, sizeof(double) * nsb) || !dxb.alloc(s, sizeof(double) * dim * m))
-        return set_error(ctx, INTI_ERR_NOMEM, "adjoint: allocation failed");
-    INTI_HIP(ctx, hipMemcpyAsync(dc.p, hc.data(), sizeof(double2) * m, hipMemcpyHostToDevice, s));
-    INTI_HIP(ctx, hipMemcpyAsync(dsg.p, hs.data(), sizeof(double2) * n, hipMemcpyHostToDevice, s));
+    if (sigma_bar)
+        if (int rc = op_transpose_correction(op)) return rc;
+    double2 *dc, *dsg;
+    double *dpart, *dsb, *dyb, *dnb, *dwb, *dkp, *dxb;
+    Arena mem(ctx);
+    mem.add(&dc, sizeof(double2) * m);
+    mem.add(&dsg, sizeof(double2) * n);
+    mem.add(&dpart, part_bytes);
+    mem.add(&dsb, sizeof(double) * (cplx ? 2 : 1) * n);
+    mem.add(&dyb, sizeof(double) * dim * n);
+    mem.add(&dnb, sizeof(double) * dim * n);
+    mem.add(&dwb, sizeof(double) * n);
+    mem.add(&dkp, sizeof(double) * nsb);
+    mem.add(&dxb, sizeof(double) * dim * m);
+    if (int rc = mem.commit()) return rc;
+    INTI_HIP(ctx, hipMemcpyAsync(dc, hc.data(), sizeof(double2) * m, hipMemcpyHostToDevice, s));
+    INTI_HIP(ctx, hipMemcpyAsync(dsg, hs.data(), sizeof(double2) * n, hipMemcpyHostToDevice, s));
 
     AdjArgs a;
     a.m = m; a.n = n;
     a.tx = op->trg->coords; a.sx = op->src->coords; a.sn = op->src->normals; a.sw = op->src->weights;
-    a.c = (const double2 *)dc.p; a.sig = (const double2 *)dsg.p;
-    a.part = (double2 *)dpart.p;
+    a.c = dc; a.sig = dsg;
+    a.part = (double2 *)dpart;
     a.p = p;
     AdjOut o;
     o.m = m; o.n = n; o.dim = dim; o.cplx = cplx;
-    o.part = (const double2 *)dpart.p; o.c = (const double2 *)dc.p; o.sig = (const double2 *)dsg.p;
+    o.part = (const double2 *)dpart; o.c = dc; o.sig = dsg;
     o.sw = op->src->weights;
     o.sn = op->src->normals;
-    o.sigma_bar = (double *)dsb.p; o.ybar = (double *)dyb.p; o.nbar = (double *)dnb.p;
-    o.wbar = (double *)dwb.p; o.kpart = (double *)dkp.p; o.xbar = (double *)dxb.p;
-    o.partr = (const double *)dpart.p;
+    o.sigma_bar = dsb; o.ybar = dyb; o.nbar = dnb;
+    o.wbar = dwb; o.kpart = dkp; o.xbar = dxb;
+    o.partr = dpart;
 
     if (fsym) {
         AdjSymArgs sa;
         sa.n = n;
         sa.xy = op->src->coords; sa.nrm = op->src->normals; sa.w = op->src->weights;
-        sa.c = (const double2 *)dc.p; sa.sig = (const double2 *)dsg.p;
-        sa.part = (double *)dpart.p; sa.kpart = (double *)dkp.p;
+        sa.c = dc; sa.sig = dsg;
+        sa.part = dpart; sa.kpart = dkp;
         sa.ntiles = symT;
         sa.distinct = op->src->distinct ? 1 : 0;
         sa.comb = comb ? 1 : 0;
@@ -1139,21 +1138,21 @@ int op_adjoint(Op *op, const double *ubar, const double *sigma, double *sigma_ba
     // corrected operator: sigma_bar also gets corr^H ubar and conj(identity) ubar
     if (sigma_bar && op->corr) {
         hipLaunchKernelGGL(k_adj_corr, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, op->corr_tptr,
-                           op->corr_trow, op->corr_tperm, op->corr->val, cplx, (const double2 *)dc.p,
-                           (double *)dsb.p);
+                           op->corr_trow, op->corr_tperm, op->corr->val, cplx, dc,
+                           dsb);
         INTI_HIP(ctx, hipGetLastError());
     }
     std::vector<double> kp(nsb);
-    if (sigma_bar) INTI_HIP(ctx, hipMemcpyAsync(sigma_bar, dsb.p, sizeof(double) * (cplx ? 2 : 1) * n, hipMemcpyDeviceToHost, s));
-    if (ybar) INTI_HIP(ctx, hipMemcpyAsync(ybar, dyb.p, sizeof(double) * dim * n, hipMemcpyDeviceToHost, s));
-    if (nbar) INTI_HIP(ctx, hipMemcpyAsync(nbar, dnb.p, sizeof(double) * dim * n, hipMemcpyDeviceToHost, s));
-    if (wbar) INTI_HIP(ctx, hipMemcpyAsync(wbar, dwb.p, sizeof(double) * n, hipMemcpyDeviceToHost, s));
+    if (sigma_bar) INTI_HIP(ctx, hipMemcpyAsync(sigma_bar, dsb, sizeof(double) * (cplx ? 2 : 1) * n, hipMemcpyDeviceToHost, s));
+    if (ybar) INTI_HIP(ctx, hipMemcpyAsync(ybar, dyb, sizeof(double) * dim * n, hipMemcpyDeviceToHost, s));
+    if (nbar) INTI_HIP(ctx, hipMemcpyAsync(nbar, dnb, sizeof(double) * dim * n, hipMemcpyDeviceToHost, s));
+    if (wbar) INTI_HIP(ctx, hipMemcpyAsync(wbar, dwb, sizeof(double) * n, hipMemcpyDeviceToHost, s));
     // combined node gradient: the symmetric pass summed the two parts; the
     // two-pass path adds the target part on the host
     std::vector<double> xsep(comb && !fsym ? (size_t)dim * m : 0);
     if (xbar && !(comb && fsym))
-        INTI_HIP(ctx, hipMemcpyAsync(comb ? xsep.data() : xbar, dxb.p, sizeof(double) * dim * m, hipMemcpyDeviceToHost, s));
-    if (kbar) INTI_HIP(ctx, hipMemcpyAsync(kp.data(), dkp.p, sizeof(double) * nsb, hipMemcpyDeviceToHost, s));
+        INTI_HIP(ctx, hipMemcpyAsync(comb ? xsep.data() : xbar, dxb, sizeof(double) * dim * m, hipMemcpyDeviceToHost, s));
+    if (kbar) INTI_HIP(ctx, hipMemcpyAsync(kp.data(), dkp, sizeof(double) * nsb, hipMemcpyDeviceToHost, s));
     INTI_HIP(ctx, hipStreamSynchronize(s));
     for (size_t q = 0; q < xsep.size(); ++q) ybar[q] += xsep[q];
     if (sigma_bar && m == n) adjoint_identity(op, cplx, n, ubar, sigma_bar);

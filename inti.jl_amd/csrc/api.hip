@@ -45,6 +45,33 @@ int ctx_scratch(Ctx *ctx, int slot, size_t bytes, void **ptr) {
     return INTI_OK;
 }
 
+Arena::~Arena() {
+    if (!live) return;
+    (void)hipStreamSynchronize(ctx->stream);
+    if (own) (void)hipFree(own);
+}
+
+int Arena::commit() {
+    size_t total = 0;
+    for (const Cut &c : cuts) total += (c.bytes + 255) / 256 * 256;
+    void *at = nullptr;
+    if (total <= kArenaKeep) {
+        if (int st = ctx_scratch(ctx, kScrTmp, total, &at)) return st;
+    } else {
+        if (hipMalloc(&own, total) != hipSuccess) {
+            own = nullptr;
+            return set_error(ctx, INTI_ERR_NOMEM, "device allocation failed");
+        }
+        at = own;
+    }
+    live = true;
+    for (const Cut &c : cuts) {
+        *c.p = at;
+        at = (char *)at + (c.bytes + 255) / 256 * 256;
+    }
+    return INTI_OK;
+}
+
 int csr_alloc(Ctx *ctx, int64_t m, int64_t n, int64_t nnz, int cplx, Csr **out) {
     Csr *c = new inti_csr();
     c->ctx = ctx; c->m = m; c->n = n; c->nnz = nnz; c->is_complex = cplx;
@@ -76,6 +103,41 @@ void op_free_correction(Op *op) {
     for (int32_t *p : ps)
         if (p) (void)hipFree(p);
     op->corr_tptr = op->corr_trow = op->corr_tperm = nullptr;
+}
+
+// Transposed pattern of the attached correction for the adjoint's gather
+// (counting sort by column; rows stay increasing within a column). Only
+// pullbacks read it, so the first one builds it.
+int op_transpose_correction(Op *op) {
+    if (!op->corr || op->corr_tptr) return INTI_OK;
+    Ctx *ctx = op->ctx;
+    const Csr *csr = op->corr;
+    const int64_t m = csr->m, n = csr->n, nnz = csr->nnz;
+    std::vector<int32_t> rp(m + 1), ci(nnz), tptr(n + 1, 0), trow(nnz), tperm(nnz);
+    INTI_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    INTI_HIP(ctx, hipMemcpy(rp.data(), csr->rowptr, sizeof(int32_t) * (m + 1), hipMemcpyDeviceToHost));
+    if (nnz > 0) INTI_HIP(ctx, hipMemcpy(ci.data(), csr->colind, sizeof(int32_t) * nnz, hipMemcpyDeviceToHost));
+    for (int64_t q = 0; q < nnz; ++q) ++tptr[ci[q] + 1];
+    for (int64_t j = 0; j < n; ++j) tptr[j + 1] += tptr[j];
+    std::vector<int32_t> fill(tptr.begin(), tptr.end() - 1);
+    for (int64_t i = 0; i < m; ++i)
+        for (int32_t q = rp[i]; q < rp[i + 1]; ++q) {
+            const int32_t p = fill[ci[q]]++;
+            trow[p] = (int32_t)i;
+            tperm[p] = q;
+        }
+    int32_t *dt[3] = {nullptr, nullptr, nullptr};
+    const int32_t *src[3] = {tptr.data(), trow.data(), tperm.data()};
+    const size_t len[3] = {(size_t)(n + 1), (size_t)nnz, (size_t)nnz};
+    for (int t = 0; t < 3; ++t)
+        if (hipMalloc((void **)&dt[t], sizeof(int32_t) * std::max<size_t>(len[t], 1)) != hipSuccess ||
+            (len[t] && hipMemcpy(dt[t], src[t], sizeof(int32_t) * len[t], hipMemcpyHostToDevice) != hipSuccess)) {
+            for (int u = 0; u < 3; ++u)
+                if (dt[u]) (void)hipFree(dt[u]);
+            return set_error(ctx, INTI_ERR_NOMEM, "adjoint: transposed pattern allocation failed");
+        }
+    op->corr_tptr = dt[0]; op->corr_trow = dt[1]; op->corr_tperm = dt[2];
+    return INTI_OK;
 }
 
 // ------------------------------------------------------- coincident nodes
@@ -669,6 +731,12 @@ int inti_op_adjoint(inti_op *op, const double *ubar, const double *sigma, double
                       dcoefs, k_bar);
 }
 
+// *flag = 1 where two index arrays differ
+__global__ __launch_bounds__(256) void k_differ(int64_t n, const int32_t *a, const int32_t *b, int *flag) {
+    const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (q < n && a[q] != b[q]) *flag = 1;
+}
+
 // merged correction: c_new = c_old + coef * csr (same pattern), or a copy
 __global__ void k_axpy_vals(int64_t nnz, int cplx, const double *src, double cr, double ci,
                             double *dst, int accumulate) {
@@ -703,60 +771,31 @@ int inti_op_attach_correction(inti_op *op, const inti_csr *csr, double coef_re, 
         // same pattern required for an in-place merge
         bool same = op->corr->nnz == csr->nnz;
         if (same && csr->nnz > 0) {
-            std::vector<int32_t> a(csr->m + 1 + csr->nnz), b(a.size());
-            INTI_HIP(ctx, hipMemcpy(a.data(), op->corr->rowptr, sizeof(int32_t) * (csr->m + 1), hipMemcpyDeviceToHost));
-            INTI_HIP(ctx, hipMemcpy(a.data() + csr->m + 1, op->corr->colind, sizeof(int32_t) * csr->nnz, hipMemcpyDeviceToHost));
-            INTI_HIP(ctx, hipMemcpy(b.data(), csr->rowptr, sizeof(int32_t) * (csr->m + 1), hipMemcpyDeviceToHost));
-            INTI_HIP(ctx, hipMemcpy(b.data() + csr->m + 1, csr->colind, sizeof(int32_t) * csr->nnz, hipMemcpyDeviceToHost));
-            same = a == b;
+            int differ = 0, *dflag = nullptr;
+            void *scr = nullptr;
+            if (int st = ctx_scratch(ctx, kScrTmp, sizeof(int), &scr)) return st;
+            dflag = (int *)scr;
+            INTI_HIP(ctx, hipMemcpyAsync(dflag, &differ, sizeof(int), hipMemcpyHostToDevice, ctx->stream));
+            hipLaunchKernelGGL(k_differ, dim3((unsigned)((csr->m + 256) / 256)), dim3(256), 0, ctx->stream, csr->m + 1,
+                               op->corr->rowptr, csr->rowptr, dflag);
+            hipLaunchKernelGGL(k_differ, dim3((unsigned)((csr->nnz + 255) / 256)), dim3(256), 0, ctx->stream, csr->nnz,
+                               op->corr->colind, csr->colind, dflag);
+            INTI_HIP(ctx, hipGetLastError());
+            INTI_HIP(ctx, hipMemcpyAsync(&differ, dflag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+            INTI_HIP(ctx, hipStreamSynchronize(ctx->stream));
+            same = differ == 0;
         }
         if (!same)
             return set_error(ctx, INTI_ERR_UNSUPPORTED, "attach: corrections with different patterns cannot be merged");
         accumulate = 1;
     } else {
-        // transposed pattern for the adjoint's gather (counting sort by
-        // column; rows stay increasing within a column)
-        const int64_t m = csr->m, n = csr->n, nnz = csr->nnz;
-        std::vector<int32_t> rp(m + 1), ci(nnz), tptr(n + 1, 0), trow(nnz), tperm(nnz);
-        INTI_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        INTI_HIP(ctx, hipMemcpy(rp.data(), csr->rowptr, sizeof(int32_t) * (m + 1), hipMemcpyDeviceToHost));
-        if (nnz > 0) INTI_HIP(ctx, hipMemcpy(ci.data(), csr->colind, sizeof(int32_t) * nnz, hipMemcpyDeviceToHost));
-        for (int64_t q = 0; q < nnz; ++q) ++tptr[ci[q] + 1];
-        for (int64_t j = 0; j < n; ++j) tptr[j + 1] += tptr[j];
-        std::vector<int32_t> fill(tptr.begin(), tptr.end() - 1);
-        for (int64_t i = 0; i < m; ++i)
-            for (int32_t q = rp[i]; q < rp[i + 1]; ++q) {
-                const int32_t p = fill[ci[q]]++;
-                trow[p] = (int32_t)i;
-                tperm[p] = q;
-            }
-        int32_t *dt[3] = {nullptr, nullptr, nullptr};
-        const size_t tb[3] = {sizeof(int32_t) * (size_t)(n + 1), sizeof(int32_t) * (size_t)std::max<int64_t>(nnz, 1),
-                              sizeof(int32_t) * (size_t)std::max<int64_t>(nnz, 1)};
-        for (int t = 0; t < 3; ++t)
-            if (hipMalloc((void **)&dt[t], tb[t]) != hipSuccess) {
-                for (int u = 0; u < 3; ++u)
-                    if (dt[u]) (void)hipFree(dt[u]);
-                return set_error(ctx, INTI_ERR_NOMEM, "attach: transposed pattern allocation failed");
-            }
         Csr *c = nullptr;
         int st = csr_alloc(ctx, csr->m, csr->n, csr->nnz, cplx, &c);
-        if (st) {
-            for (int u = 0; u < 3; ++u) (void)hipFree(dt[u]);
-            return st;
-        }
+        if (st) return st;
         op->corr = c;
-        op->corr_tptr = dt[0]; op->corr_trow = dt[1]; op->corr_tperm = dt[2];
         INTI_HIP(ctx, hipMemcpyAsync(c->rowptr, csr->rowptr, sizeof(int32_t) * (csr->m + 1), hipMemcpyDeviceToDevice, ctx->stream));
         if (csr->nnz > 0)
             INTI_HIP(ctx, hipMemcpyAsync(c->colind, csr->colind, sizeof(int32_t) * csr->nnz, hipMemcpyDeviceToDevice, ctx->stream));
-        INTI_HIP(ctx, hipMemcpyAsync(dt[0], tptr.data(), tb[0], hipMemcpyHostToDevice, ctx->stream));
-        if (nnz > 0) {
-            INTI_HIP(ctx, hipMemcpyAsync(dt[1], trow.data(), sizeof(int32_t) * nnz, hipMemcpyHostToDevice, ctx->stream));
-            INTI_HIP(ctx, hipMemcpyAsync(dt[2], tperm.data(), sizeof(int32_t) * nnz, hipMemcpyHostToDevice, ctx->stream));
-        }
-        // the host vectors above must outlive the asynchronous uploads
-        INTI_HIP(ctx, hipStreamSynchronize(ctx->stream));
     }
     if (csr->nnz > 0) {
         hipLaunchKernelGGL(k_axpy_vals, dim3((unsigned)((csr->nnz + 255) / 256)), dim3(256), 0, ctx->stream,

@@ -580,6 +580,117 @@ int bdim_build_types(Op *opS, Op *opD, int deriv, int ntypes, const int *nq, con
     // triplets (type, element, target, node) -> (row, col), CSR pattern
     const int64_t ntri = tri_off[ntypes];
     if (ntri >= (int64_t)INT32_MAX) return set_error(ctx, INTI_ERR_SIZE, "bdim: too many triplets");
+    // ---- device buffers
+    std::vector<double> zs;
+    monopoles(src, ns, radius_mult, zs);
+    std::vector<int32_t> qt32((size_t)ntags);
+    for (size_t q = 0; q < qt32.size(); ++q) qt32[q] = (int32_t)qtags[q];
+    const int rl = 2 * dim + (opS->pde == INTI_HELMHOLTZ ? 4 : 2) * nst;
+    // source split: the fewest rounds of resident blocks per unit of work,
+    // the smaller split on ties. Every split adds nloc x nst partial sums
+    // written and read once: up to 3 when the tiles alone fill a round
+    // (partial traffic <= 3x Theta), more only for small builds
+    const int64_t ntiles = std::max<int64_t>(1, (nloc + 63) / 64);
+    const int64_t slots = (int64_t)fns.theta_occ * ctx->num_cu;
+    const int64_t want = std::max<int64_t>(3, (slots + ntiles - 1) / ntiles);
+    const int64_t max_split = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(64, want),
+                                                                     n / (64 * kThetaWaves)));
+    int64_t best = 1;
+    double best_cost = 1e300;
+    for (int64_t sp = 1; sp <= max_split; ++sp) {
+        const double rounds = (double)((ntiles * sp + slots - 1) / slots);
+        const double cost = rounds / (double)sp;
+        if (cost < best_cost * (1 - 1e-9)) { best_cost = cost; best = sp; }
+    }
+    const int split = (int)best;
+    const int64_t chunk = (n + split - 1) / split;
+    double *dzs, *drec, *ddiag, *dmu;
+    int32_t *dqt, *dglob, *dpp, *dploc, *delems, *dseg, *dperm;
+    double2 *dB0, *dB1, *dpart, *dth, *dtriS, *dtriD;
+    const size_t cb = sizeof(double2), ib = sizeof(int32_t);
+    TripletPattern pat;  // outlives the arena, which drains the uploads
+    Arena mem(ctx);
+    mem.add(&dzs, zs.size() * sizeof(double));
+    mem.add(&dqt, qt32.size() * ib);
+    mem.add(&dglob, glob.size() * ib);
+    mem.add(&dpp, pair_ptr.size() * ib);
+    mem.add(&dploc, pair_loc.size() * ib);
+    mem.add(&delems, elems.size() * ib);
+    mem.add(&dB0, cb * n * nsp);
+    mem.add(&dB1, cb * n * nsp);
+    mem.add(&dth, cb * nloc * ns);
+    mem.add(&dtriS, cb * ntri);
+    mem.add(&dtriD, cb * ntri);
+    mem.add(&ddiag, sizeof(double) * 3 * elems.size());
+    mem.add(&dseg, ib * (size_t)(ntri + 1));  // the pattern has at most ntri entries
+    mem.add(&dperm, ib * (size_t)ntri);
+    mem.add(&dmu, sizeof(double) * m);
+    mem.add(&drec, nloc > 0 ? sizeof(double) * n * rl : 0);
+    mem.add(&dpart, nloc > 0 && split > 1 ? cb * split * nst * nloc : 0);
+    if (int rc = mem.commit()) return rc;
+    hipStream_t st = ctx->stream;
+    auto up = [&](void *d, const void *h, size_t bytes) {
+        return bytes ? hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, st) : hipSuccess;
+    };
+    INTI_HIP(ctx, up(dzs, zs.data(), zs.size() * sizeof(double)));
+    INTI_HIP(ctx, up(dqt, qt32.data(), qt32.size() * ib));
+    INTI_HIP(ctx, up(dglob, glob.data(), glob.size() * ib));
+    INTI_HIP(ctx, up(dpp, pair_ptr.data(), pair_ptr.size() * ib));
+    INTI_HIP(ctx, up(dploc, pair_loc.data(), pair_loc.size() * ib));
+    INTI_HIP(ctx, up(delems, elems.data(), elems.size() * ib));
+    INTI_HIP(ctx, up(dmu, mu, sizeof(double) * m));
+
+    KParams kp = basic_params(opS->k);
+    kp.kimag = opS->kimag;
+
+    // traces
+    {
+        TraceArgs a;
+        a.n = n; a.ns = ns; a.nsp = nsp;
+        a.sx = src->coords; a.sn = src->normals; a.zs = dzs;
+        a.B0 = dB0; a.B1 = dB1;
+        a.p = kp;
+        fns.traces(a, dim3((unsigned)((n * nsp + 255) / 256)), st);
+        INTI_HIP(ctx, hipGetLastError());
+    }
+    // Theta: pack the per-source records, then the sum (and the reduction of
+    // its partial sums when the sources are split over several blocks)
+    if (nloc > 0) {
+        ThetaPackArgs pa;
+        pa.n = n; pa.ns = ns; pa.nsp = nsp; pa.nst = nst; pa.rl = rl;
+        pa.sx = src->coords; pa.sn = src->normals; pa.sw = src->weights;
+        pa.B0 = dB0; pa.B1 = dB1;
+        pa.rec = drec;
+        basic_post(opS->pde, dim, deriv ? INTI_ADL : INTI_SL, opS->k, pa.psr, pa.psi);
+        basic_post(opS->pde, dim, deriv ? INTI_HS : INTI_DL, opS->k, pa.pdr, pa.pdi);
+        fns.pack(pa, dim3((unsigned)((n * (nst + 1) + 255) / 256)), st);
+        INTI_HIP(ctx, hipGetLastError());
+        ThetaArgs a;
+        a.m = m; a.n = n; a.nloc = nloc;
+        a.ns = ns; a.rl = rl; a.split = split; a.chunk = chunk;
+        a.glob = dglob;
+        a.tx = trg->coords; a.tn = trg->normals;
+        a.rec = drec;
+        a.zs = dzs; a.mu = dmu;
+        a.part = dpart;
+        a.theta = dth;
+        a.p = kp;
+        fns.theta(a, dim3((unsigned)(ntiles * split)), st);
+        INTI_HIP(ctx, hipGetLastError());
+        if (split > 1) {
+            ThetaRedArgs r;
+            r.m = m; r.nloc = nloc; r.ns = ns; r.nst = nst; r.split = split;
+            r.glob = dglob;
+            r.tx = trg->coords; r.tn = trg->normals; r.zs = dzs;
+            r.mu = dmu;
+            r.part = dpart;
+            r.theta = dth;
+            r.p = kp;
+            fns.reduce(r, dim3((unsigned)((nloc * ns + 255) / 256)), st);
+            INTI_HIP(ctx, hipGetLastError());
+        }
+    }
+    // the CSR pattern, on the host while the GPU works on Theta
     std::vector<int32_t> tri_row(ntri), tri_col(ntri);
     for (int t = 0; t < ntypes; ++t) {
         const int64_t *qt = qtags + tag_off[t];
@@ -592,133 +703,26 @@ int bdim_build_types(Op *opS, Op *opD, int deriv, int ntypes, const int *nq, con
                     tri_col[q] = (int32_t)qt[r + (int64_t)nq[t] * e];
                 }
     }
-    TripletPattern pat;
     build_pattern(m, tri_row, tri_col, pat);
     const std::vector<int32_t> &rowptr = pat.rowptr, &colind = pat.colind, &seg = pat.seg, &perm = pat.perm;
     const int64_t nnz = (int64_t)colind.size();
 
-    // ---- device buffers
-    std::vector<double> zs;
-    monopoles(src, ns, radius_mult, zs);
-    std::vector<int32_t> qt32((size_t)ntags);
-    for (size_t q = 0; q < qt32.size(); ++q) qt32[q] = (int32_t)qtags[q];
-    DevBuf dzs, dqt, dglob, dpp, dploc, delems, dB0, dB1, dpart, drec, dth, dtriS, dtriD, ddiag, dseg, dperm, dmu;
-    const size_t cb = sizeof(double2);
-    INTI_ALLOC(ctx, dzs, zs.size() * sizeof(double));
-    INTI_ALLOC(ctx, dqt, qt32.size() * sizeof(int32_t));
-    INTI_ALLOC(ctx, dglob, glob.size() * sizeof(int32_t));
-    INTI_ALLOC(ctx, dpp, pair_ptr.size() * sizeof(int32_t));
-    INTI_ALLOC(ctx, dploc, pair_loc.size() * sizeof(int32_t));
-    INTI_ALLOC(ctx, delems, elems.size() * sizeof(int32_t));
-    INTI_ALLOC(ctx, dB0, cb * n * nsp);
-    INTI_ALLOC(ctx, dB1, cb * n * nsp);
-    INTI_ALLOC(ctx, dth, cb * nloc * ns);
-    INTI_ALLOC(ctx, dtriS, cb * ntri);
-    INTI_ALLOC(ctx, dtriD, cb * ntri);
-    INTI_ALLOC(ctx, ddiag, sizeof(double) * 3 * elems.size());
-    INTI_ALLOC(ctx, dseg, sizeof(int32_t) * seg.size());
-    INTI_ALLOC(ctx, dperm, sizeof(int32_t) * perm.size());
-    INTI_ALLOC(ctx, dmu, sizeof(double) * m);
-    hipStream_t st = ctx->stream;
-    auto up = [&](void *d, const void *h, size_t bytes) {
-        return bytes ? hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, st) : hipSuccess;
-    };
-    INTI_HIP(ctx, up(dzs.p, zs.data(), zs.size() * sizeof(double)));
-    INTI_HIP(ctx, up(dqt.p, qt32.data(), qt32.size() * sizeof(int32_t)));
-    INTI_HIP(ctx, up(dglob.p, glob.data(), glob.size() * sizeof(int32_t)));
-    INTI_HIP(ctx, up(dpp.p, pair_ptr.data(), pair_ptr.size() * sizeof(int32_t)));
-    INTI_HIP(ctx, up(dploc.p, pair_loc.data(), pair_loc.size() * sizeof(int32_t)));
-    INTI_HIP(ctx, up(delems.p, elems.data(), elems.size() * sizeof(int32_t)));
-    INTI_HIP(ctx, up(dseg.p, seg.data(), seg.size() * sizeof(int32_t)));
-    INTI_HIP(ctx, up(dperm.p, perm.data(), perm.size() * sizeof(int32_t)));
-    INTI_HIP(ctx, up(dmu.p, mu, sizeof(double) * m));
-
-    KParams kp = basic_params(opS->k);
-    kp.kimag = opS->kimag;
-
-    // traces
-    {
-        TraceArgs a;
-        a.n = n; a.ns = ns; a.nsp = nsp;
-        a.sx = src->coords; a.sn = src->normals; a.zs = (const double *)dzs.p;
-        a.B0 = (double2 *)dB0.p; a.B1 = (double2 *)dB1.p;
-        a.p = kp;
-        fns.traces(a, dim3((unsigned)((n * nsp + 255) / 256)), st);
-        INTI_HIP(ctx, hipGetLastError());
-    }
-    // Theta: pack the per-source records, then the sum (and the reduction of
-    // its partial sums when the sources are split over several blocks)
-    if (nloc > 0) {
-        const int pk = opS->pde == INTI_HELMHOLTZ ? 4 : 2;
-        const int rl = 2 * dim + pk * nst;
-        INTI_ALLOC(ctx, drec, sizeof(double) * n * rl);
-        ThetaPackArgs pa;
-        pa.n = n; pa.ns = ns; pa.nsp = nsp; pa.nst = nst; pa.rl = rl;
-        pa.sx = src->coords; pa.sn = src->normals; pa.sw = src->weights;
-        pa.B0 = (const double2 *)dB0.p; pa.B1 = (const double2 *)dB1.p;
-        pa.rec = (double *)drec.p;
-        basic_post(opS->pde, dim, deriv ? INTI_ADL : INTI_SL, opS->k, pa.psr, pa.psi);
-        basic_post(opS->pde, dim, deriv ? INTI_HS : INTI_DL, opS->k, pa.pdr, pa.pdi);
-        fns.pack(pa, dim3((unsigned)((n * (nst + 1) + 255) / 256)), st);
-        INTI_HIP(ctx, hipGetLastError());
-        // source split: the fewest rounds of resident blocks per unit of work,
-        // the smaller split on ties. Every split adds nloc x nst partial sums
-        // written and read once: up to 3 when the tiles alone fill a round
-        // (partial traffic <= 3x Theta), more only for small builds
-        const int64_t ntiles = (nloc + 63) / 64;
-        const int64_t slots = (int64_t)fns.theta_occ * ctx->num_cu;
-        const int64_t want = std::max<int64_t>(3, (slots + ntiles - 1) / ntiles);
-        const int64_t max_split = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(64, want),
-                                                                         n / (64 * kThetaWaves)));
-        int64_t best = 1;
-        double best_cost = 1e300;
-        for (int64_t sp = 1; sp <= max_split; ++sp) {
-            const double rounds = (double)((ntiles * sp + slots - 1) / slots);
-            const double cost = rounds / (double)sp;
-            if (cost < best_cost * (1 - 1e-9)) { best_cost = cost; best = sp; }
-        }
-        const int split = (int)best;
-        const int64_t chunk = (n + split - 1) / split;
-        if (split > 1) INTI_ALLOC(ctx, dpart, sizeof(double2) * split * nst * nloc);
-        ThetaArgs a;
-        a.m = m; a.n = n; a.nloc = nloc;
-        a.ns = ns; a.rl = rl; a.split = split; a.chunk = chunk;
-        a.glob = (const int32_t *)dglob.p;
-        a.tx = trg->coords; a.tn = trg->normals;
-        a.rec = (const double *)drec.p;
-        a.zs = (const double *)dzs.p; a.mu = (const double *)dmu.p;
-        a.part = (double2 *)dpart.p;
-        a.theta = (double2 *)dth.p;
-        a.p = kp;
-        fns.theta(a, dim3((unsigned)(ntiles * split)), st);
-        INTI_HIP(ctx, hipGetLastError());
-        if (split > 1) {
-            ThetaRedArgs r;
-            r.m = m; r.nloc = nloc; r.ns = ns; r.nst = nst; r.split = split;
-            r.glob = (const int32_t *)dglob.p;
-            r.tx = trg->coords; r.tn = trg->normals; r.zs = (const double *)dzs.p;
-            r.mu = (const double *)dmu.p;
-            r.part = (const double2 *)dpart.p;
-            r.theta = (double2 *)dth.p;
-            r.p = kp;
-            fns.reduce(r, dim3((unsigned)((nloc * ns + 255) / 256)), st);
-            INTI_HIP(ctx, hipGetLastError());
-        }
-    }
+    INTI_HIP(ctx, up(dseg, seg.data(), ib * seg.size()));
+    INTI_HIP(ctx, up(dperm, perm.data(), ib * perm.size()));
     // batched QR + LS, one launch per element type
     for (int t = 0; t < ntypes; ++t) {
         const int64_t nel = elems_off[t + 1] - elems_off[t];
         if (nel == 0) continue;
         LsArgs a;
         a.n = n; a.nloc = nloc; a.nq = nq[t]; a.ns = ns;
-        a.elems = (const int32_t *)delems.p + elems_off[t];
-        a.qtags = (const int32_t *)dqt.p + tag_off[t];
-        a.pair_ptr = (const int32_t *)dpp.p + el_off[t];
-        a.pair_loc = (const int32_t *)dploc.p + pair_off[t];
-        a.B0 = (const double2 *)dB0.p; a.B1 = (const double2 *)dB1.p; a.ldb = n;
-        a.theta = (const double2 *)dth.p;
-        a.triS = (double2 *)dtriS.p + tri_off[t]; a.triD = (double2 *)dtriD.p + tri_off[t];
-        a.diag = (double *)ddiag.p + 3 * elems_off[t];
+        a.elems = delems + elems_off[t];
+        a.qtags = dqt + tag_off[t];
+        a.pair_ptr = dpp + el_off[t];
+        a.pair_loc = dploc + pair_off[t];
+        a.B0 = dB0; a.B1 = dB1; a.ldb = n;
+        a.theta = dth;
+        a.triS = dtriS + tri_off[t]; a.triD = dtriD + tri_off[t];
+        a.diag = ddiag + 3 * elems_off[t];
         hipLaunchKernelGGL(k_ls, dim3((unsigned)nel), dim3(64), 0, st, a);
         INTI_HIP(ctx, hipGetLastError());
     }
@@ -738,17 +742,17 @@ int bdim_build_types(Op *opS, Op *opD, int deriv, int ntypes, const int *nq, con
     {
         Gather1Args g;
         g.nnz = nnz;
-        g.seg = (const int32_t *)dseg.p; g.perm = (const int32_t *)dperm.p;
+        g.seg = dseg; g.perm = dperm;
         g.cplx = cplx;
-        g.tri = (const double2 *)dtriS.p; g.val = cS->val; g.sign = -1.0;
+        g.tri = dtriS; g.val = cS->val; g.sign = -1.0;
         launch_gather1(g, st);
-        g.tri = (const double2 *)dtriD.p; g.val = cD->val; g.sign = 1.0;
+        g.tri = dtriD; g.val = cD->val; g.sign = 1.0;
         launch_gather1(g, st);
         if (hipGetLastError() != hipSuccess) return fail(set_error(ctx, INTI_ERR_HIP, "bdim: gather launch failed"));
     }
     std::vector<double> dg(3 * elems.size());
     if (!dg.empty() &&
-        hipMemcpyAsync(dg.data(), ddiag.p, sizeof(double) * dg.size(), hipMemcpyDeviceToHost, st) != hipSuccess)
+        hipMemcpyAsync(dg.data(), ddiag, sizeof(double) * dg.size(), hipMemcpyDeviceToHost, st) != hipSuccess)
         return fail(set_error(ctx, INTI_ERR_HIP, "bdim: diag copy failed"));
     if (hipStreamSynchronize(st) != hipSuccess)
         return fail(set_error(ctx, INTI_ERR_HIP, "bdim: kernel execution failed"));

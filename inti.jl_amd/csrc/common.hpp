@@ -73,7 +73,7 @@ struct Op {
     double cid[2] = {0, 0};          // identity coefficient (square ops)
     const Quad *trg = nullptr, *src = nullptr;
     Csr *corr = nullptr;  // owned merged correction (may be null)
-    // the correction's transposed pattern (built at the first attach; the
+    // the correction's transposed pattern (built by the first pullback; the
     // pattern never changes while attached): column j's entries are
     // corr_trow[p] / corr->val[corr_tperm[p]] for p in [corr_tptr[j],
     // corr_tptr[j+1]), rows increasing. The adjoint gathers through it.
@@ -101,6 +101,33 @@ int set_error(Ctx *ctx, int code, const std::string &msg);
 enum { kScrPartial = 0, kScrX = 1, kScrY = 2, kScrTmp = 3 };
 int ctx_scratch(Ctx *ctx, int slot, size_t bytes, void **ptr);
 
+// The device temporaries of one call: sizes are added, then one buffer is cut
+// into them (256-byte aligned). Up to kArenaKeep bytes the buffer is the
+// context's kScrTmp scratch, kept for the next call; beyond, an allocation of
+// this call alone. The arena drains the stream when it goes (an error return
+// may leave copies from the call's host vectors queued: declare those first).
+class Arena {
+  public:
+    explicit Arena(Ctx *c) : ctx(c) {}
+    Arena(const Arena &) = delete;
+    Arena &operator=(const Arena &) = delete;
+    ~Arena();
+    template <typename T>
+    void add(T **p, size_t bytes) { cuts.push_back({(void **)p, bytes}); }
+    int commit();
+
+  private:
+    struct Cut {
+        void **p;
+        size_t bytes;
+    };
+    Ctx *ctx;
+    std::vector<Cut> cuts;
+    void *own = nullptr;
+    bool live = false;
+};
+constexpr size_t kArenaKeep = size_t(512) << 20;
+
 // ------------------------------------------------------- kernel dispatchers
 struct DirectLaunch {
     const Op *op;
@@ -126,6 +153,7 @@ int refine_solve(Op *op_hi, Op *op_lo, Op *prec, const double *b, double *x, int
                  double *relres);
 int launch_assemble(const Op *op, double *out_dev);
 void op_free_correction(Op *op);
+int op_transpose_correction(Op *op);  // builds corr_tptr ... once
 int op_adjoint(Op *op, const double *ubar, const double *sigma, double *sigma_bar, double *ybar,
                double *nbar, double *wbar, double *xbar, const double *dcoefs, double *kbar);
 
