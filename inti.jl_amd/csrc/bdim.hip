@@ -67,9 +67,7 @@ __global__ __launch_bounds__(256) void k_traces(TraceArgs a) {
 // quarter of the block's sources; the quarters are added in LDS in wave
 // order (deterministic). With one source chunk (split = 1) the block writes
 // Theta itself, mu G included; otherwise partial sums go to `part` and
-// k_theta_reduce adds them. (Measured at 63,480 nodes, 3D Helmholtz, ns = 18:
-// 4 waves and 3 source chunks 32.3 ms, 24 chunks 29.6 ms; 3 waves and one
-// chunk, all 992 blocks nominally resident, 46.6 ms.)
+// k_theta_reduce adds them (the split: bdim_build_types).
 constexpr int kThetaWaves = 4;
 constexpr int kThetaRed = 8;  // doubles per lane per LDS reduction round
 
@@ -586,21 +584,36 @@ int bdim_build_types(Op *opS, Op *opD, int deriv, int ntypes, const int *nq, con
     std::vector<int32_t> qt32((size_t)ntags);
     for (size_t q = 0; q < qt32.size(); ++q) qt32[q] = (int32_t)qtags[q];
     const int rl = 2 * dim + (opS->pde == INTI_HELMHOLTZ ? 4 : 2) * nst;
-    // source split: the fewest rounds of resident blocks per unit of work,
-    // the smaller split on ties. Every split adds nloc x nst partial sums
-    // written and read once: up to 3 when the tiles alone fill a round
-    // (partial traffic <= 3x Theta), more only for small builds
+    // Source split. Block b takes chunk b % split, and the blocks are dealt to
+    // the 8 XCDs round robin, so with a multiple of 8 every XCD reads only its
+    // share of the records, which its L2 and scalar caches then hold: the
+    // scalar loads of the records are what the kernel waits for beside its
+    // FMAs. 8 chunks, 16 where 8 leave the chip short of blocks (below one and
+    // a half rounds of resident ones). Whole builds, ms, with the split that
+    // fills the fewest rounds (at most 3 where the tiles fill one) / 8:
+    // 3D Helmholtz 4,320 nodes 0.57 / 0.50 (16), 12,000: 1.83 / 1.70, 30,720:
+    // 8.80 / 7.29, 63,480: 33.2 / 28.4, 33,800 with 30 monopoles 18.8 / 15.4;
+    // 3D Laplace 30,720: 3.20 / 3.00, 63,480: 13.3 / 10.5.
+    // Other splits (4, 6, 12) lie between; two targets per lane, twice the
+    // FMAs per record, changed these by under 3 %. Builds too small for 8
+    // chunks, or with more partial sums than 2 GiB, take the fewest rounds of
+    // resident blocks per unit of work, the smaller split on ties, up to 3
+    // when the tiles alone fill a round.
     const int64_t ntiles = std::max<int64_t>(1, (nloc + 63) / 64);
     const int64_t slots = (int64_t)fns.theta_occ * ctx->num_cu;
-    const int64_t want = std::max<int64_t>(3, (slots + ntiles - 1) / ntiles);
-    const int64_t max_split = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(64, want),
-                                                                     n / (64 * kThetaWaves)));
-    int64_t best = 1;
-    double best_cost = 1e300;
-    for (int64_t sp = 1; sp <= max_split; ++sp) {
-        const double rounds = (double)((ntiles * sp + slots - 1) / slots);
-        const double cost = rounds / (double)sp;
-        if (cost < best_cost * (1 - 1e-9)) { best_cost = cost; best = sp; }
+    const int64_t most = std::min<int64_t>(64, n / (64 * kThetaWaves));
+    const size_t per_split = sizeof(double2) * (size_t)nst * (size_t)nloc;
+    int64_t best = 2 * ntiles * 8 < 3 * slots && most >= 16 ? 16 : 8;
+    if (most < 8 || best * per_split > (size_t(2) << 30)) {
+        const int64_t want = std::max<int64_t>(3, (slots + ntiles - 1) / ntiles);
+        const int64_t max_split = std::max<int64_t>(1, std::min(want, most));
+        double best_cost = 1e300;
+        best = 1;
+        for (int64_t sp = 1; sp <= max_split; ++sp) {
+            const double rounds = (double)((ntiles * sp + slots - 1) / slots);
+            const double cost = rounds / (double)sp;
+            if (cost < best_cost * (1 - 1e-9)) { best_cost = cost; best = sp; }
+        }
     }
     const int split = (int)best;
     const int64_t chunk = (n + split - 1) / split;
