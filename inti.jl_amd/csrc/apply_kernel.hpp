@@ -509,7 +509,8 @@ __global__ __launch_bounds__(kApplyBS) void k_apply_row(RowArgs a) {
         nt[d] = g.tn ? g.tn[d * g.tstride + ic] : 0.0;
     }
     double sr = 0.0, si = 0.0;
-    constexpr int UNR = CPLX && DIM == 2 ? 1 : 2;
+    // two pairs in flight but for the 2D Helmholtz and logarithm kernels
+    constexpr int UNR = DIM == 2 && (CPLX || KIND == INTI_SL || KIND == INTI_COMB_SD) ? 1 : 2;
 #pragma unroll UNR
     for (int64_t j = tid / tb; j < g.n; j += nsl) {
         double y[DIM], ny[DIM];

@@ -62,11 +62,59 @@ __device__ __forceinline__ double rcpv(double x) {
     if constexpr (MIXED) return (double)__builtin_amdgcn_rcpf((float)x);
     else return rcp64(x);
 }
-// natural logarithm
+// a b + c as one three-address v_fma_f64 with the addend in scalar registers:
+// Horner steps with coefficients from tables. Left to itself the compiler
+// makes each such step a copy of the coefficient into vector registers (two
+// moves) and a two-address v_fmac_f64; the copies were 96 of the 260 vector
+// instructions of a Hankel evaluation beyond x = 5 and 136 of 304 below.
+__device__ __forceinline__ double fma_sc(double a, double b, double c) {
+    double r;
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "s"(c));
+    return r;
+}
+
+// R(z) / z of log((1 + s) / (1 - s)) = 2 s + s R(z), z = s^2, for |s| <=
+// (sqrt 2 - 1) / (sqrt 2 + 1): minimax polynomial of degree 6 (Remez, 50
+// digits; largest error 3.1e-16, 4.5e-18 of the logarithm).
+constexpr double kLogR[7] = {0x1.5555555555558p-1, 0x1.999999999522ep-2, 0x1.2492492e02bd5p-2, 0x1.c71c62d1afefbp-3,
+                             0x1.7462b9bf192ccp-3, 0x1.39fdc6eb9e894p-3, 0x1.2b5f15b8214eep-3};
+// ln 2 = hi + lo, hi with 11 trailing zero bits (k hi is exact)
+constexpr double kLn2Hi = 0x1.62e42fefa3800p-1, kLn2Lo = 0x1.ef35793c76730p-45;
+
+// Natural logarithm of a positive finite x in FP64: x = 2^k (1 + f), sqrt(1/2)
+// <= 1 + f < sqrt 2; with s = f / (2 + f), log(1 + f) = 2 s + s R(s^2). The
+// quotient's rounding error is carried (sl) and k ln 2 + 2 s is added without
+// one, so the result is within 0.54 ulp (20,000 samples in exact arithmetic).
+// About 40 instructions in the place of the 75 of the library's equally exact
+// one: 2D Laplace SL and the Hankel functions below x = 5 spent most of a pair
+// on it. (The plain form f - s (f - R), ten instructions less, is off by up to
+// 1.1 ulp, which the ill-conditioned DIM weights of 2D Laplace show.)
+__device__ __forceinline__ double log64(double x) {
+    double m = __builtin_amdgcn_frexp_mant(x);
+    int e = __builtin_amdgcn_frexp_exp(x);
+    const bool low = m < 0x1.6a09e667f3bcdp-1;
+    m = low ? m + m : m;
+    e = low ? e - 1 : e;
+    const double f = m - 1.0, k = (double)e;
+    const double d = 2.0 + f, dl = f - (d - 2.0);  // 2 + f = d + dl
+    const double r = rcp64(d);
+    const double s = f * r;
+    const double sl = __builtin_fma(-s, dl, __builtin_fma(-s, d, f)) * r;
+    const double z = s * s;
+    double p = kLogR[6];
+#pragma unroll
+    for (int i = 5; i >= 0; --i) p = fma_sc(p, z, kLogR[i]);
+    const double a = k * kLn2Hi;
+    const double h = __builtin_fma(2.0, s, a), l = __builtin_fma(2.0, s, a - h);
+    const double t = __builtin_fma(2.0, sl, __builtin_fma(k, kLn2Lo, l));
+    return h + __builtin_fma(s * z, p, t);
+}
+
+// natural logarithm of x >= 0
 template <bool MIXED>
 __device__ __forceinline__ double logv(double x) {
     if constexpr (MIXED) return (double)(__builtin_amdgcn_logf((float)x) * 0.69314718f);
-    else return log(x);
+    else return x < __builtin_inf() ? log64(x) : x;  // infinity and NaN stay
 }
 
 // Taylor coefficients of sin(2 pi f) / f and cos(2 pi f) in z = f^2:
@@ -122,6 +170,25 @@ __device__ __forceinline__ void sincos_rev64_vop3(double u, double &s, double &c
     double pc = kCosRev[8];
 #pragma unroll
     for (int k = 7; k >= 0; --k) pc = fma_vop3(pc, z, kCosRev[k]);
+    const double S = f * ps, C = pc;
+    const int qi = (int)q & 3;
+    const double s0 = (qi & 1) ? C : S;
+    const double c0 = (qi & 1) ? S : C;
+    s = (qi & 2) ? -s0 : s0;
+    c = ((qi ^ (qi >> 1)) & 1) ? -c0 : c0;
+}
+
+// The same with the coefficients as scalar addends (fma_sc).
+__device__ __forceinline__ void sincos_rev64_sc(double u, double &s, double &c) {
+    const double q = __builtin_rint(4.0 * u);
+    const double f = __builtin_fma(-0.25, q, u);
+    const double z = f * f;
+    double ps = kSinRev[7];
+#pragma unroll
+    for (int k = 6; k >= 0; --k) ps = fma_sc(ps, z, kSinRev[k]);
+    double pc = kCosRev[8];
+#pragma unroll
+    for (int k = 7; k >= 0; --k) pc = fma_sc(pc, z, kCosRev[k]);
     const double S = f * ps, C = pc;
     const int qi = (int)q & 3;
     const double s0 = (qi & 1) ? C : S;
@@ -192,7 +259,7 @@ template <int N>
 __device__ __forceinline__ double horner_p(ConstF64Ptr c, double u) {
     double s = c[N - 1];
 #pragma unroll
-    for (int i = N - 2; i >= 0; --i) s = __builtin_fma(s, u, c[i]);
+    for (int i = N - 2; i >= 0; --i) s = fma_sc(s, u, c[i]);
     return s;
 }
 
@@ -205,7 +272,7 @@ __device__ __forceinline__ void hankel01_f64(double x, double &h0r, double &h0i,
         double u = 0.25 * x * x;
         double a0 = horner_p<18>(tb->a0, u), a1 = horner_p<18>(tb->a1, u);
         double b0 = horner_p<18>(tb->b0, u), b1 = horner_p<18>(tb->b1, u);
-        double L = log(0.5 * x);
+        double L = log64(0.5 * x);
         double ix = rcp64(x);
         double J0 = a0, J1 = 0.5 * x * a1;
         h0r = J0;
@@ -213,16 +280,16 @@ __device__ __forceinline__ void hankel01_f64(double x, double &h0r, double &h0i,
         h1r = J1;
         h1i = -kTwoOverPi * ix + kTwoOverPi * L * J1 - (0.5 / kPi) * x * b1;
     } else {
-        double ix = rcp64(x);
+        const double y = rsq64(x), ix = y * y;
         double t = (HK_F64_XS * HK_F64_XS) * ix * ix;
         double P0 = horner_p<7>(tb->p0n, t) * rcp64(horner_p<7>(tb->p0d, t));
         double Q0 = horner_p<7>(tb->q0n, t) * rcp64(horner_p<7>(tb->q0d, t)) * ix;
         double P1 = horner_p<7>(tb->p1n, t) * rcp64(horner_p<7>(tb->p1d, t));
         double Q1 = horner_p<7>(tb->q1n, t) * rcp64(horner_p<7>(tb->q1d, t)) * ix;
-        double amp = kSqrt2OverPi * rsq64(x);
+        double amp = kSqrt2OverPi * y;
         // phase x - pi/4 in revolutions: sin/cos(2 pi (x/(2 pi) - 1/8))
         double s, c;
-        sincos_rev64(__builtin_fma(x, kInv2Pi, -0.125), s, c);
+        sincos_rev64_sc(__builtin_fma(x, kInv2Pi, -0.125), s, c);
         // H0 = amp (P0 + i Q0)(c + i s); H1 = amp (P1 + i Q1)(s - i c)
         h0r = amp * (P0 * c - Q0 * s);
         h0i = amp * (P0 * s + Q0 * c);

@@ -145,17 +145,18 @@ constexpr size_t kSymSmallBytes = size_t(512) << 20;
 // therefore cut into one-wave blocks of 64 nodes (one target per lane, below
 // 12 waves per CU of 128-node blocks, about 10,000 nodes) or 128 nodes (two
 // targets per lane, below 72 tile pairs of 256 nodes per CU, about 49,000).
-// The 2D Helmholtz pairs take 64 wherever the partial sums allow: their
-// Hankel evaluation branches on the argument, and one wave without barriers
-// waits for no other wave's branch. Measured, us per apply with 256 / 128 /
+// The 2D Helmholtz pairs take 64 wherever the partial sums allow (in mixed
+// precision up to 24 tile pairs per CU, about 28,000 nodes): their Hankel
+// evaluation branches on the argument, and one wave without barriers waits
+// for no other wave's branch. Measured, us per apply with 256 / 128 /
 // 64-node tiles (before: one direction below 8,200 nodes):
 //   3D Helmholtz CF FP64   4,320: 101 / 57 / 44 (one direction 83)
 //                         12,000: 253 / 213 / 206    24,000: 837 / 734 / 750
 //                         40,000: 2001 / 1926 / 2084 63,480: 4826 / 4894 / 5320
 //   3D Laplace SL FP64     4,320: 55 / 22 / 19 (29)  8,500: 58 / 42 / 41
 //                         24,000: 214 / 188 / 216    63,480: 1125 / 1171 / 1463
-//   2D Helmholtz CF FP64   6,006: 479 / 437 / 251 (500)  30,720: 4222 / 4114 / 3869
-//   2D Helmholtz CF mixed  6,006: 123 / 120 / 82 (146)   40,000: 2011 / 2032 / 1999
+//   2D Helmholtz CF FP64   6,006: 333 / - / 179 (328)  30,720: 2592 / - / 2583
+//   2D Helmholtz CF mixed  6,006: 123 / - / 82 (146)   40,000: 1989 / - / 2019
 // Sums of 256 nodes or fewer run in one direction (k_apply_row). An explicit
 // group keeps tiles of 256. Beyond kSymMaxBytes of partial sums the groups of
 // 2 and 4 tiles halve and quarter them.
@@ -169,7 +170,9 @@ bool plan_sym(const Op *op, int kind, SymPlan &P) {
         const int64_t t128 = tiles(128), t256 = tiles(kSymBS), cu = op->ctx->num_cu;
         const bool helm2 = op->pde == INTI_HELMHOLTZ && op->dim == 2;
         int tile = kSymBS;
-        if (helm2 || t128 * (t128 + 1) / 2 < 12 * cu) tile = 64;
+        const bool mixed = op->precision == INTI_MIXED;
+        if (helm2 ? !mixed || t256 * (t256 + 1) / 2 < 24 * cu : t128 * (t128 + 1) / 2 < 12 * cu) tile = 64;
+        else if (helm2) tile = kSymBS;
         else if (t256 * (t256 + 1) / 2 < 72 * cu) tile = 128;
         if (tile < kSymBS && (size_t)tiles(tile) * (size_t)n * es <= kSymSmallBytes) {
             P = SymPlan{tile, 1, tiles(tile), tiles(tile)};
@@ -195,7 +198,7 @@ bool plan_sym(const Op *op, int kind, SymPlan &P) {
 // more than the loads: few pairs. Against the symmetric sum it is faster up
 // to about 1,800 nodes (3D Helmholtz CF 1,280: 15 / 20 us, 3,000: 41 / 33;
 // 3D Laplace SL 1,280: 8 / 11, 3,000: 23 / 15) and, for 2D Helmholtz, up to
-// 3,400 (CF 3,000: 96 / 150; 4,320: 205 / 171); against the one-direction sum
+// 3,400 (CF 3,000: 73 / 102; 4,320: 145 / 125); against the one-direction sum
 // with its second kernel up to 2,400 (Laplace 2,000: 11 / 20; 3,000: 23 / 21)
 // and 3,800 nodes (3D Helmholtz CF 3,000: 40 / 59; 4,320: 85 / 83). The 2D
 // Helmholtz kernels keep it at any size once 4 m threads per CU are in

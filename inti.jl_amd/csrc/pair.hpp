@@ -560,7 +560,16 @@ __device__ __forceinline__ void pair_value(const double *r, const double *nx, co
     static_assert(KIND <= INTI_HS || KIND == INTI_FF_SL || KIND == INTI_FF_DL,
                   "combined kinds carry their post factor in KParams");
     double rr, ri, pr, pi;
-    pair_raw<PDE, DIM, KIND, false>(r, nx, ny, p, rr, ri);
+    if constexpr (PDE == INTI_LAPLACE && DIM == 2 && KIND == INTI_SL) {
+        // the DIM least squares are made of these values and amplify their
+        // last bits by up to 1e9: the library's logarithm, rounded almost
+        // always correctly, and not log64
+        const double d2 = dotv<2>(r, r);
+        rr = mask(d2 > kSamePointTol2, log(fmax(d2, kClampD2)));
+        ri = 0.0;
+    } else {
+        pair_raw<PDE, DIM, KIND, false>(r, nx, ny, p, rr, ri);
+    }
     basic_post(PDE, DIM, KIND, p.k, pr, pi);
     kr = pr * rr - pi * ri;
     ki = pr * ri + pi * rr;
