@@ -257,7 +257,8 @@ int inti_batch_bdim_build(inti_batch *batch, int nq, const int64_t *ne, const in
 /* add coef * csr (problem-local indices, n_p x n_p) to problem p */
 int inti_batch_attach_correction(inti_batch *batch, int p, const inti_csr *csr,
                                  double coef_re, double coef_im);
-/* source chunk length of a work item (0 = 2048) and persistent grid size
+/* source chunk length of a work item (0 = automatic: 2048 for large batches,
+ * 512 or 256 for smaller ones) and persistent grid size
  * (0 = 4 workgroups per CU) */
 int inti_batch_set_launch(inti_batch *batch, int64_t chunk_len, int grid);
 /* y = alpha A x + beta y; device (leading dimensions >= ntot) or host */

@@ -39,7 +39,7 @@ struct Batch {
     int32_t *row2p = nullptr;
     double *cid_d = nullptr;
     // launch plan
-    int64_t chunk_len = 2048;  // source chunk length of a work item
+    int64_t chunk_len = 0;  // source chunk length of a work item; 0 = automatic (batch_chunk)
     int grid = 0;              // persistent grid; 0 = 4 blocks per CU
     bool planned = false;
     BatchItem *items = nullptr;
@@ -76,10 +76,41 @@ static BatchFn pick_batch(int pde, int dim, int kind, int mixed, int nr) {
 }
 
 // ------------------------------------------------------------------ plan
+// Automatic chunk length. An item is 256 targets against a chunk, and about
+// two blocks per CU are resident (the 16-density kernels hold 200 registers),
+// so a batch of few items leaves the last of them alone on the chip: chunks
+// of 2048 sources need eight items per resident block, chunks of 512 one;
+// smaller batches are cut finest. Shorter chunks cost partial sums (16
+// densities x n per chunk, at most 1 GiB here before 2048 is taken back).
+// us per apply of 16 densities with 256 / 512 / 1024 / 2048, mixed: 48 2D
+// problems of 79,088 nodes in all 901 / 817 / 918 / 1046; 48 of 37,824: 234 /
+// 230 / 340 / 500; 12 of 17,328: 187 / 225 / 257 / 461; 3 of 1,884: 72 / 127 /
+// 180 / 278; 200 of 325,424: 3264 / 3166 / 3148 / 3213 (FP64 6617 / 6635 /
+// 6728 / 6873).
+static int64_t batch_chunk(const Batch *B) {
+    const int64_t slots = 2LL * B->ctx->num_cu;
+    auto plan = [&](int64_t L, int64_t &items, int64_t &sums) {
+        items = sums = 0;
+        for (int p = 0; p < B->nprob; ++p) {
+            const int64_t n = B->off[p + 1] - B->off[p];
+            items += (n + kApplyBS - 1) / kApplyBS * ((n + L - 1) / L);
+            sums += 16 * n * ((n + L - 1) / L);
+        }
+    };
+    int64_t items, sums;
+    plan(2048, items, sums);
+    if (items >= 8 * slots) return 2048;
+    plan(512, items, sums);
+    const int64_t cw = B->pde == INTI_HELMHOLTZ ? 2 : 1;
+    if (sums * cw * (int64_t)sizeof(double) > (int64_t(1) << 30)) return 2048;
+    return items >= slots ? 512 : 256;
+}
+
 static int batch_plan(Batch *B) {
     if (B->planned) return INTI_OK;
     Ctx *ctx = B->ctx;
-    const int64_t L = std::max<int64_t>(kApplyBS, (B->chunk_len + kApplyBS - 1) / kApplyBS * kApplyBS);
+    const int64_t want = B->chunk_len > 0 ? B->chunk_len : batch_chunk(B);
+    const int64_t L = std::max<int64_t>(kApplyBS, (want + kApplyBS - 1) / kApplyBS * kApplyBS);
     B->hprobs.assign(B->nprob, BatchProb{});
     struct It { BatchItem w; int64_t cost; };
     std::vector<It> its;
@@ -1243,9 +1274,8 @@ int inti_batch_set_launch(inti_batch *B, int64_t chunk_len, int grid) {
     if (!B) return INTI_ERR_ARG;
     BREQ(B->ctx, chunk_len >= 0 && grid >= 0, "batch_set_launch: negative value");
     BLOCK(B->ctx);
-    const int64_t c = chunk_len > 0 ? chunk_len : 2048;
-    if (c != B->chunk_len) B->planned = false;
-    B->chunk_len = c;
+    if (chunk_len != B->chunk_len) B->planned = false;
+    B->chunk_len = chunk_len;
     B->grid = grid;
     return INTI_OK;
 }
