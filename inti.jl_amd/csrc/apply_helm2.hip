@@ -4,7 +4,7 @@
 
 namespace inti {
 ApplyFn apply_pick_helm2(int kind, int mixed, int nr) { return apply_pick_pd<INTI_HELMHOLTZ, 2>(kind, mixed, nr); }
-RowFn row_pick_helm2(int kind, int mixed) { return row_pick_pd<INTI_HELMHOLTZ, 2>(kind, mixed); }
+RowFn row_pick_helm2(int kind, int mixed, int nr) { return row_pick_pd<INTI_HELMHOLTZ, 2>(kind, mixed, nr); }
 BatchFn batch_pick_helm2(int kind, int mixed, int nr) { return batch_pick_pd<INTI_HELMHOLTZ, 2>(kind, mixed, nr); }
 SymFn sym_pick_helm2(int kind, int mixed, int tile, int G) { return sym_pick_pd<INTI_HELMHOLTZ, 2>(kind, mixed, tile, G); }
 SymFn sym_trans_pick_helm2(int kind, int tile, int G) { return sym_trans_pick_pd<INTI_HELMHOLTZ, 2>(kind, tile, G); }

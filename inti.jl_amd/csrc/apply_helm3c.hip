@@ -10,5 +10,5 @@ ApplyFn apply_pick_helm3c(int kind, int nr) {
     if (nr == 16) return apply_kind<kHelmCK, 3, false, 16>(kind);
     return nullptr;
 }
-RowFn row_pick_helm3c(int kind) { return row_kind<kHelmCK, 3, false>(kind); }
+RowFn row_pick_helm3c(int kind, int nr) { return row_nr<kHelmCK, 3, false>(kind, nr); }
 }  // namespace inti

@@ -478,8 +478,8 @@ __device__ __forceinline__ void reduce_epilogue(const ReduceArgs &a, int64_t i, 
 }
 
 // ------------------------------------------------------ small sums, one launch
-// One right-hand side of few targets in one launch: a block takes tb targets
-// (4 ... 64, a power of two) and 256 / tb threads share each target's
+// NR (1 or 4) right-hand sides of few targets in one launch: a block takes tb
+// targets (4 ... 64, a power of two) and 256 / tb threads share each target's
 // sources, thread t of a target taking sources t, t + 256 / tb, ... read
 // straight from memory (consecutive threads read consecutive sources). The
 // threads' sums are added in a fixed order (lanes by a butterfly, then the
@@ -492,11 +492,11 @@ struct RowArgs {
     int tb;
 };
 
-template <int PDE, int DIM, int KIND, bool MIXED>
+template <int PDE, int DIM, int KIND, bool MIXED, int NR>
 __global__ __launch_bounds__(kApplyBS) void k_apply_row(RowArgs a) {
     constexpr bool CPLX = PDE != INTI_LAPLACE;
     constexpr int NW = kApplyBS / 64;
-    __shared__ double2 s_w[NW][64];
+    __shared__ double2 s_w[NW][NR][64];
     const ApplyArgs &g = a.s;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int tb = a.tb, t = tid & (tb - 1), nsl = kApplyBS / tb;
@@ -508,7 +508,9 @@ __global__ __launch_bounds__(kApplyBS) void k_apply_row(RowArgs a) {
         xt[d] = g.tx[d * g.tstride + ic];
         nt[d] = g.tn ? g.tn[d * g.tstride + ic] : 0.0;
     }
-    double sr = 0.0, si = 0.0;
+    double sr[NR], si[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) sr[r] = si[r] = 0.0;
     // two pairs in flight but for the 2D Helmholtz and logarithm kernels
     constexpr int UNR = DIM == 2 && (CPLX || KIND == INTI_SL || KIND == INTI_COMB_SD) ? 1 : 2;
 #pragma unroll UNR
@@ -522,30 +524,43 @@ __global__ __launch_bounds__(kApplyBS) void k_apply_row(RowArgs a) {
         const double w = g.sw[j];
         double kr, ki;
         pair_raw_xy<PDE, DIM, KIND, MIXED>(xt, nt, y, ny, g.p, kr, ki);
-        if constexpr (CPLX) {
-            const double2 xv = reinterpret_cast<const double2 *>(g.x)[j];
-            const double qr = w * xv.x, qi = w * xv.y;
-            sr = __builtin_fma(kr, qr, sr);
-            sr = __builtin_fma(-ki, qi, sr);
-            si = __builtin_fma(kr, qi, si);
-            si = __builtin_fma(ki, qr, si);
-        } else {
-            sr = __builtin_fma(kr, w * g.x[j], sr);
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            if constexpr (CPLX) {
+                const double2 xv = reinterpret_cast<const double2 *>(g.x)[j + r * g.ldx];
+                const double qr = w * xv.x, qi = w * xv.y;
+                sr[r] = __builtin_fma(kr, qr, sr[r]);
+                sr[r] = __builtin_fma(-ki, qi, sr[r]);
+                si[r] = __builtin_fma(kr, qi, si[r]);
+                si[r] = __builtin_fma(ki, qr, si[r]);
+            } else {
+                sr[r] = __builtin_fma(kr, w * g.x[j + r * g.ldx], sr[r]);
+            }
         }
     }
     for (int o = tb; o < 64; o *= 2) {
-        sr += __shfl_xor(sr, o);
-        if constexpr (CPLX) si += __shfl_xor(si, o);
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            sr[r] += __shfl_xor(sr[r], o);
+            if constexpr (CPLX) si[r] += __shfl_xor(si[r], o);
+        }
     }
-    if (lane < tb) s_w[wave][lane] = make_double2(sr, si);
+    if (lane < tb) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r) s_w[wave][r][lane] = make_double2(sr[r], si[r]);
+    }
     __syncthreads();
-    if (tid < tb && i < g.m) {
+    // row t of right-hand side r = tid / tb
+    const int r = tid / tb;
+    if (r < NR && i < g.m) {
+        double2 v = s_w[0][r][t];
 #pragma unroll
         for (int w = 1; w < NW; ++w) {
-            sr += s_w[w][tid].x;
-            si += s_w[w][tid].y;
+            v.x += s_w[w][r][t].x;
+            v.y += s_w[w][r][t].y;
         }
-        reduce_epilogue<CPLX>(a.e, i, a.e.x, a.e.y, sr, si);
+        constexpr int CW = CPLX ? 2 : 1;
+        reduce_epilogue<CPLX>(a.e, i, a.e.x + CW * (int64_t)r * a.e.ldx, a.e.y + CW * (int64_t)r * a.e.ldy, v.x, v.y);
     }
 }
 
@@ -620,34 +635,39 @@ static int apply_launcher(const ApplyArgs *a, dim3 grid, hipStream_t s) {
 
 using RowFn = void (*)(const RowArgs &, dim3, hipStream_t);
 
-template <int PDE, int DIM, int KIND, bool MIXED>
+template <int PDE, int DIM, int KIND, bool MIXED, int NR>
 static void row_launcher(const RowArgs &a, dim3 grid, hipStream_t s) {
-    hipLaunchKernelGGL((k_apply_row<PDE, DIM, KIND, MIXED>), grid, dim3(kApplyBS), 0, s, a);
+    hipLaunchKernelGGL((k_apply_row<PDE, DIM, KIND, MIXED, NR>), grid, dim3(kApplyBS), 0, s, a);
 }
 
-template <int PDE, int DIM, bool MIXED>
+template <int PDE, int DIM, bool MIXED, int NR>
 static RowFn row_kind(int kind) {
     switch (kind) {
-        case INTI_SL: return row_launcher<PDE, DIM, INTI_SL, MIXED>;
-        case INTI_DL: return row_launcher<PDE, DIM, INTI_DL, MIXED>;
-        case INTI_ADL: return row_launcher<PDE, DIM, INTI_ADL, MIXED>;
-        case INTI_HS: return row_launcher<PDE, DIM, INTI_HS, MIXED>;
-        case INTI_COMB_SD: return row_launcher<PDE, DIM, INTI_COMB_SD, MIXED>;
-        case INTI_COMB_AH: return row_launcher<PDE, DIM, INTI_COMB_AH, MIXED>;
+        case INTI_SL: return row_launcher<PDE, DIM, INTI_SL, MIXED, NR>;
+        case INTI_DL: return row_launcher<PDE, DIM, INTI_DL, MIXED, NR>;
+        case INTI_ADL: return row_launcher<PDE, DIM, INTI_ADL, MIXED, NR>;
+        case INTI_HS: return row_launcher<PDE, DIM, INTI_HS, MIXED, NR>;
+        case INTI_COMB_SD: return row_launcher<PDE, DIM, INTI_COMB_SD, MIXED, NR>;
+        case INTI_COMB_AH: return row_launcher<PDE, DIM, INTI_COMB_AH, MIXED, NR>;
     }
     if constexpr (PDE == INTI_HELMHOLTZ) {
         switch (kind) {
-            case INTI_FF_SL: return row_launcher<PDE, DIM, INTI_FF_SL, MIXED>;
-            case INTI_FF_DL: return row_launcher<PDE, DIM, INTI_FF_DL, MIXED>;
-            case INTI_FF_COMB: return row_launcher<PDE, DIM, INTI_FF_COMB, MIXED>;
+            case INTI_FF_SL: return row_launcher<PDE, DIM, INTI_FF_SL, MIXED, NR>;
+            case INTI_FF_DL: return row_launcher<PDE, DIM, INTI_FF_DL, MIXED, NR>;
+            case INTI_FF_COMB: return row_launcher<PDE, DIM, INTI_FF_COMB, MIXED, NR>;
         }
     }
     return nullptr;
 }
 
+// nr in {1, 4}
+template <int PDE, int DIM, bool MIXED>
+static RowFn row_nr(int kind, int nr) {
+    return nr == 1 ? row_kind<PDE, DIM, MIXED, 1>(kind) : nr == 4 ? row_kind<PDE, DIM, MIXED, 4>(kind) : nullptr;
+}
 template <int PDE, int DIM>
-static RowFn row_pick_pd(int kind, int mixed) {
-    return mixed ? row_kind<PDE, DIM, true>(kind) : row_kind<PDE, DIM, false>(kind);
+static RowFn row_pick_pd(int kind, int mixed, int nr) {
+    return mixed ? row_nr<PDE, DIM, true>(kind, nr) : row_nr<PDE, DIM, false>(kind, nr);
 }
 
 // transposed FP64 sums (one right-hand side) of the kinds with a pullback
@@ -751,10 +771,10 @@ ApplyFn apply_pick_helm2(int kind, int mixed, int nr);
 ApplyFn apply_pick_helm3(int kind, int mixed, int nr);
 ApplyFn apply_pick_helm3c(int kind, int nr);  // complex wavenumber, FP64
 
-RowFn row_pick_lap2(int kind, int mixed);
-RowFn row_pick_lap3(int kind, int mixed);
-RowFn row_pick_helm2(int kind, int mixed);
-RowFn row_pick_helm3(int kind, int mixed);
-RowFn row_pick_helm3c(int kind);  // complex wavenumber, FP64
+RowFn row_pick_lap2(int kind, int mixed, int nr);
+RowFn row_pick_lap3(int kind, int mixed, int nr);
+RowFn row_pick_helm2(int kind, int mixed, int nr);
+RowFn row_pick_helm3(int kind, int mixed, int nr);
+RowFn row_pick_helm3c(int kind, int nr);  // complex wavenumber, FP64
 
 }  // namespace inti

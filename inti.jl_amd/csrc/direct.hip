@@ -111,12 +111,12 @@ static ApplyFn pick_apply(int pde, int dim, int kind, int mixed, int nr) {
     return nullptr;
 }
 
-static RowFn pick_row(int pde, int dim, int kind, int mixed) {
-    if (pde == INTI_LAPLACE && dim == 2) return row_pick_lap2(kind, mixed);
-    if (pde == INTI_LAPLACE && dim == 3) return row_pick_lap3(kind, mixed);
-    if (pde == INTI_HELMHOLTZ && dim == 2) return row_pick_helm2(kind, mixed);
-    if (pde == INTI_HELMHOLTZ && dim == 3) return row_pick_helm3(kind, mixed);
-    if (pde == kHelmCK && dim == 3 && !mixed) return row_pick_helm3c(kind);
+static RowFn pick_row(int pde, int dim, int kind, int mixed, int nr) {
+    if (pde == INTI_LAPLACE && dim == 2) return row_pick_lap2(kind, mixed, nr);
+    if (pde == INTI_LAPLACE && dim == 3) return row_pick_lap3(kind, mixed, nr);
+    if (pde == INTI_HELMHOLTZ && dim == 2) return row_pick_helm2(kind, mixed, nr);
+    if (pde == INTI_HELMHOLTZ && dim == 3) return row_pick_helm3(kind, mixed, nr);
+    if (pde == kHelmCK && dim == 3 && !mixed) return row_pick_helm3c(kind, nr);
     return nullptr;
 }
 
@@ -190,8 +190,8 @@ bool plan_sym(const Op *op, int kind, SymPlan &P) {
     return false;
 }
 
-// Targets per block of the one-launch sum (k_apply_row) for a single
-// right-hand side of m targets and n sources, 0 where another sum is taken.
+// Targets per block of the one-launch sum (k_apply_row) for nr right-hand
+// sides of m targets and n sources, 0 where another sum is taken.
 // Four targets per block and 64 threads per target keep every thread's
 // source chain short; it reads each source's data once per 16 threads instead
 // of staging it, so it pays where launches, barriers and an idle chip cost
@@ -206,11 +206,20 @@ bool plan_sym(const Op *op, int kind, SymPlan &P) {
 // of the Hankel functions' branch more often than one of 64 targets (CF FP64
 // 12,000: 1264 / 1337 us, 30,720: 7785 / 8235). The chain of a thread is
 // bounded (n <= 8,192) where the targets alone do not fill the chip.
-static int plan_row(const Op *op, int64_t m, int64_t n, bool sym) {
-    if (op->split > 0 || n <= 0) return 0;
-    if (sym && op->sym == 2) return 0;
+// Four right-hand sides reuse each pair value, so the staged kernel overtakes
+// earlier: 2,200 nodes in 3D Helmholtz (DL 640: 8 / 36 us, 2,000: 27 / 37,
+// 2,600: 46 / 39), 1,800 for Laplace (3D SL 1,280: 12 / 18, 2,000: 18 / 18)
+// and 3,700 in 2D Helmholtz (CF FP64 1,280: 26 / 140, 3,200: 106 / 156, mixed
+// 3,200: 62 / 72, 4,320: 104 / 90). 16 go to the matrix-core kernel at once.
+static int plan_row(const Op *op, int64_t m, int64_t n, bool sym, int nr) {
+    if (op->split > 0 || n <= 0 || nr > 4) return 0;
     const double pairs = (double)m * (double)n;
     const bool lap = op->pde == INTI_LAPLACE, helm2 = op->pde == INTI_HELMHOLTZ && op->dim == 2;
+    if (nr == 4) {
+        const double lim4 = helm2 ? 3700.0 : lap ? 1800.0 : 2200.0;
+        return n <= 8192 && pairs <= lim4 * lim4 ? 4 : 0;
+    }
+    if (sym && op->sym == 2) return 0;
     if (helm2 && !sym && m >= 4LL * op->ctx->num_cu) return 4;
     const double lim = sym ? (helm2 ? 3400.0 : 1800.0) : (helm2 ? 3400.0 : lap ? 2400.0 : 3800.0);
     return n <= 8192 && pairs <= lim * lim ? 4 : 0;
@@ -262,10 +271,20 @@ KParams op_params(const Op *op, int *eff_kind) {
 // then share a chunk in their L2); an explicit split (inti_op_set_launch)
 // replaces it. Without one, the plan then looks at splits from half to twice
 // the base (multiples of 8 from 8 on) with chunks of whole LDS source tiles of
-// the kernel (256, 128 or 64 sources for 1, 4 or 16 right-hand sides) and
-// takes the one with the least rounds x chunk, where blocks run in rounds of
-// `cap` resident blocks (occupancy x CUs): a grid just past a multiple of cap
-// leaves its last round nearly empty.
+// the kernel and takes the one with the least rounds x chunk, where blocks run
+// in rounds of `cap` resident blocks (occupancy x CUs): a grid just past a
+// multiple of cap leaves its last round nearly empty.
+// With 4 or 16 right-hand sides one or two blocks keep a CU busy, so the time
+// follows the blocks of the fullest CU x chunk whatever the occupancy, and all
+// splits from half to four times the base are looked at, down to one LDS tile
+// (128 or 64 sources) per chunk; a shorter chunk would cost as much as a whole
+// one (the inner loop runs over padding). kChunkCost, in sources, stands for a
+// block's start and its partial sums; where a lone block per CU waits on its
+// own chains (4 columns, and the 2D Helmholtz kernels) it costs as much as a
+// second one beside it. Against rounds of resident blocks:
+// 4 columns, 3D Helmholtz DL, 4,320 nodes 100 -> 75 us, 9,000: 280 -> 224; 16
+// columns, 1,700 nodes 79 -> 31, 4,320: 115 -> 102.
+constexpr int64_t kChunkCost = 8;
 static void plan_split(const Op *op, int64_t m, int64_t n, ApplyFn fn, int nr, int &split, int64_t &chunk) {
     const int64_t ntiles = (m + kApplyBS - 1) / kApplyBS;
     const int64_t stiles = (n + kApplyBS - 1) / kApplyBS;
@@ -279,12 +298,13 @@ static void plan_split(const Op *op, int64_t m, int64_t n, ApplyFn fn, int nr, i
     if (op->split <= 0 && fn && n > 0) {
         const int64_t gran = nr == 16 ? kMfmaTT : nr == 4 ? ApplyTile<4>::TT : ApplyTile<1>::TT;
         const int64_t gtiles = (n + gran - 1) / gran;
-        const double cap = (double)fn(nullptr, dim3(0), nullptr) * op->ctx->num_cu;
-        auto cost_of = [&](int64_t c) { return std::ceil((double)(ntiles * ((n + c - 1) / c)) / cap) * (double)c; };
-        double best = cost_of(chunk);  // the base plan stays unless a candidate beats it
-        for (int64_t s = std::max<int64_t>(1, s0 / 2); s <= std::min(2 * s0, gtiles); s += s < 8 ? 1 : 8) {
-            const int64_t c = (gtiles + s - 1) / s * gran;
-            const double cost = cost_of(c);
+        const int64_t cus = op->ctx->num_cu, cap = nr == 1 ? (int64_t)fn(nullptr, dim3(0), nullptr) * cus : cus;
+        const int64_t lone = nr == 4 || (nr == 16 && op->pde == INTI_HELMHOLTZ && op->dim == 2) ? 1 : 0;
+        const int64_t over = nr == 1 ? 0 : kChunkCost, smax = std::min((nr == 1 ? 2 : 4) * s0, gtiles);
+        auto cost_of = [&](int64_t c) { return ((ntiles * ((n + c - 1) / c) + cap - 1) / cap + lone) * (c + over); };
+        int64_t best = cost_of(chunk);  // the base plan stays unless a candidate beats it
+        for (int64_t s = std::max<int64_t>(1, s0 / 2); s <= smax; s += s < 8 || nr > 1 ? 1 : 8) {
+            const int64_t c = (gtiles + s - 1) / s * gran, cost = cost_of(c);
             if (cost < best) {
                 best = cost;
                 chunk = c;
@@ -296,7 +316,7 @@ static void plan_split(const Op *op, int64_t m, int64_t n, ApplyFn fn, int nr, i
 }
 
 // scratch of the column blocks (16, 4, 1) a call of nrhs columns uses
-int apply_reserve(const Op *op, int nrhs) {
+int apply_reserve(const Op *op, int nrhs, bool rows) {
     const int cw = op_is_complex(op) ? 2 : 1;
     const int64_t m = op->trg->n, n = op->src->n;
     int kind = op->kind;
@@ -307,11 +327,13 @@ int apply_reserve(const Op *op, int nrhs) {
         if (nrhs < nr) continue;
         if (nr == 1) {
             const bool sym = plan_sym(op, kind, sp);
-            if (plan_row(op, m, n, sym)) continue;
+            if (rows && plan_row(op, m, n, sym, nr)) continue;
             if (sym) {
                 bytes = std::max(bytes, sizeof(double) * cw * (size_t)sp.S * (size_t)n);
                 continue;
             }
+        } else if (rows && plan_row(op, m, n, false, nr)) {
+            continue;
         }
         int split;
         int64_t chunk;
@@ -333,8 +355,12 @@ int launch_apply(const DirectLaunch &L) {
     const KParams kp = op_params(op, &kind);
     const bool given = L.part != nullptr;
     double *part = L.part;
+    // the one-launch sum writes rows of y while others still read x: an apply
+    // in place keeps the sums whose second kernel writes y
+    const double *xend = L.x + cw * ((int64_t)(L.nrhs - 1) * L.ldx + n), *yend = L.y + cw * ((int64_t)(L.nrhs - 1) * L.ldy + m);
+    const bool rows = L.x >= yend || L.y >= xend;
     if (!given) {
-        int st = apply_reserve(op, L.nrhs);
+        int st = apply_reserve(op, L.nrhs, rows);
         if (st) return st;
         void *scr = nullptr;
         st = ctx_scratch(ctx, kScrPartial, 0, &scr);
@@ -363,8 +389,8 @@ int launch_apply(const DirectLaunch &L) {
         ra.cr = op->cid[0]; ra.ci = op->cid[1];
         ra.pr = kp.postr; ra.pi = kp.posti;
         ra.has_id = (op->cid[0] != 0.0 || op->cid[1] != 0.0);
-        const int tb = nr == 1 ? plan_row(op, m, n, sym) : 0;
-        RowFn rfn = tb ? pick_row(op_kernel_pde(op), op->dim, kind, op->precision == INTI_MIXED) : nullptr;
+        const int tb = rows ? plan_row(op, m, n, sym, nr) : 0;
+        RowFn rfn = tb ? pick_row(op_kernel_pde(op), op->dim, kind, op->precision == INTI_MIXED, nr) : nullptr;
         ApplyFn fn = rfn || (sym && nr == 1) ? nullptr : pick_apply(op_kernel_pde(op), op->dim, kind, op->precision == INTI_MIXED, nr);
         int split = 1;
         int64_t chunk = n;

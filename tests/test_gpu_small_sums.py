@@ -3,6 +3,8 @@
 oracle (FP64 <= 1e-12, the bar of every direct sum; mixed <= 1e-6) on all rows
 of the small sizes and on the first and last rows of the large ones. The
 densities are random, the nodes a spiral on the sphere or an ellipse."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -97,3 +99,46 @@ def test_repeat_is_bit_identical(inti, n):
     A = inti.IntegralOperator(_kernel(inti, 1, 3, 4)[0], Q, Q)
     x = np.random.default_rng(5).normal(size=n) + 0j
     assert np.array_equal(A @ x, A @ x)
+
+
+# four right-hand sides at once: around the largest one-launch sums, the plans
+# of one LDS tile per chunk, and a remainder of single columns
+@pytest.mark.parametrize("pde,dim,kind", [(0, 2, 1), (0, 3, 3), (1, 2, 4), (1, 3, 1)])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("n,nrhs", [(1, 4), (67, 5), (1801, 4), (2201, 4), (3701, 6), (2900, 16)])
+def test_columns(inti, oracle, pde, dim, kind, precision, n, nrhs):
+    Q = _nodes(inti, dim, n)
+    K, coefs = _kernel(inti, pde, dim, kind)
+    A = inti.IntegralOperator(K, Q, Q, precision=precision)
+    rng = np.random.default_rng(11)
+    x = rng.normal(size=(n, nrhs)) + (1j * rng.normal(size=(n, nrhs)) if pde else 0.0)
+    y = A @ x
+    for r in range(nrhs):
+        ref = oracle.matvec(pde, dim, kind, 7.3 if pde else 0.0, Q, Q, np.ascontiguousarray(x[:, r]), coefs=coefs)
+        err, size = np.linalg.norm(y[:, r] - ref), np.linalg.norm(ref)
+        say(f"[gpu] pde {pde} dim {dim} kind {kind} {precision} n={n} column {r}: {err:.2e} of {size:.2e}")
+        assert err <= (1e-12 if precision == "fp64" else 1e-6) * size
+
+
+# an apply in place: no row may be written while others still read it
+@pytest.mark.parametrize("nrhs", [1, 4])
+def test_in_place(inti, nrhs):
+    n = 1500
+    Q = _nodes(inti, 3, n)
+    A = inti.IntegralOperator(_kernel(inti, 1, 3, 4)[0], Q, Q)
+    rng = np.random.default_rng(13)
+    x = rng.normal(size=(nrhs, n)) + 1j * rng.normal(size=(nrhs, n))
+    ctx, lib, hip = A.ctx, A.ctx.lib, ctypes.CDLL("libamdhip64.so")
+    one, zero = (ctypes.c_double * 2)(1.0, 0.0), (ctypes.c_double * 2)(0.0, 0.0)
+    dx = ctypes.c_void_p()
+    assert hip.hipMalloc(ctypes.byref(dx), ctypes.c_size_t(x.nbytes)) == 0
+    assert hip.hipMemcpy(dx, x.ctypes.data_as(ctypes.c_void_p), ctypes.c_size_t(x.nbytes), 1) == 0
+    ctx.check(lib.inti_op_apply_device(A.handle, nrhs, dx, n, dx, n, one, zero))
+    ctx.synchronize()
+    y = np.empty_like(x)
+    assert hip.hipMemcpy(y.ctypes.data_as(ctypes.c_void_p), dx, ctypes.c_size_t(x.nbytes), 2) == 0
+    assert hip.hipFree(dx) == 0
+    ref = np.stack([A @ x[r] for r in range(nrhs)])
+    err = np.linalg.norm(y - ref) / np.linalg.norm(ref)
+    say(f"[gpu] in place, {nrhs} columns: {err:.2e}")
+    assert err <= 1e-12
