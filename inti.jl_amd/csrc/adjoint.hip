@@ -477,6 +477,7 @@ __global__ __launch_bounds__(256) void k_adj_trg_reduce(AdjOut o) {
 // kbar += Re(sc gk). The waves' sums for a sub-tile are added in LDS in wave
 // order; one partial slot per (node, tile) as in the forward sum;
 // deterministic.
+constexpr int kAdjSmallTile = 128;
 struct AdjSymArgs {
     int64_t n;
     const double *xy, *nrm, *w;
@@ -484,6 +485,7 @@ struct AdjSymArgs {
     double *part;   // S x NR x n
     double *kpart;  // one per block
     int64_t ntiles;
+    int tile;       // nodes per tile: kSymBS or kAdjSmallTile
     int distinct;   // no two nodes within twice the coincidence tolerance
     int comb;       // one node gradient, source and target parts summed
     int chik;       // 3D combined field with c0 = -i k, c1 = 1, dc0 = -i, dc1 = 0
@@ -535,19 +537,19 @@ __device__ __forceinline__ void lds_add(double *a, double v) {
 // asked for by passing the same output for both): NR = 2 DIM + 2 sums
 // [S0 (2), G (DIM), N (DIM)] instead of 3 DIM + 2, and each pair adds its
 // difference g1 - g2 once to each node.
-template <int PDE, int DIM, int KIND, bool COMB, bool CHIK = false>
-__global__ __launch_bounds__(kSymBS) __attribute__((amdgpu_waves_per_eu(COMB ? 3 : 1))) void k_adj_sym(AdjSymArgs A) {
+template <int PDE, int DIM, int KIND, bool COMB, bool CHIK, int TS>
+__global__ __launch_bounds__(TS) __attribute__((amdgpu_waves_per_eu(COMB ? 3 : 1))) void k_adj_sym(AdjSymArgs A) {
     constexpr int NR = COMB ? 2 * DIM + 2 : 3 * DIM + 2;
     constexpr double OSC = CHIK ? kInv4Pi : 1.0;  // see adj_radial (CHIK)
-    constexpr int NW = kSymBS / 64;
+    constexpr int NW = TS / 64;
     constexpr int iY = 2, iX = COMB ? 2 : 2 + DIM, iN = COMB ? 2 + DIM : 2 + 2 * DIM;
-    __shared__ double s_x[DIM][kSymBS], s_n[DIM][kSymBS];
-    __shared__ double2 s_c[kSymBS], s_s[kSymBS];
+    __shared__ double s_x[DIM][TS], s_n[DIM][TS];
+    __shared__ double2 s_c[TS], s_s[TS];
     // per-wave sums of the current 64-source sub-tile: at step s lane l adds
     // to source (l + s) mod 64, so the 64 lanes of a wave add to 64 different
     // addresses and each address receives its terms in step order
     __shared__ double s_acc[NW][NR][64];
-    __shared__ double s_k[kSymBS];
+    __shared__ double s_k[TS];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int64_t a, b;
     sym_item(blockIdx.x, A.ntiles, a, b);
@@ -556,11 +558,11 @@ __global__ __launch_bounds__(kSymBS) __attribute__((amdgpu_waves_per_eu(COMB ? 3
     const AdjParams &p = A.p;
     double xi[DIM], ni[DIM];
     double2 ci, si;
-    adj_sym_node<DIM>(A, a * kSymBS + tid, xi, ni, ci, si);
+    adj_sym_node<DIM>(A, a * TS + tid, xi, ni, ci, si);
     {
         double xj[DIM], nj[DIM];
         double2 cj, sj;
-        adj_sym_node<DIM>(A, b * kSymBS + tid, xj, nj, cj, sj);
+        adj_sym_node<DIM>(A, b * TS + tid, xj, nj, cj, sj);
 #pragma unroll
         for (int d = 0; d < DIM; ++d) { s_x[d][tid] = xj[d]; s_n[d][tid] = nj[d]; }
         s_c[tid] = cj;
@@ -572,7 +574,7 @@ __global__ __launch_bounds__(kSymBS) __attribute__((amdgpu_waves_per_eu(COMB ? 3
     double kb = 0.0;
     // unrolled: the sub-tile offsets u * 64 become immediate LDS offsets
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < NW; ++u) {
         __syncthreads();  // the previous sub-tile's sums have been read; s_x.. are written
         double *acc = &s_acc[wave][0][0];
 #pragma unroll
@@ -654,7 +656,7 @@ __global__ __launch_bounds__(kSymBS) __attribute__((amdgpu_waves_per_eu(COMB ? 3
         // lane l owns tile row u * 64 + l (= tid), also the row of its own
         // sums below
         if (wave == u) {
-            const int64_t j = b * kSymBS + tid;
+            const int64_t j = b * TS + tid;
             if (j < n) {
 #pragma unroll
                 for (int r = 0; r < NR; ++r) {
@@ -669,7 +671,7 @@ __global__ __launch_bounds__(kSymBS) __attribute__((amdgpu_waves_per_eu(COMB ? 3
     // source tile b's sums went to slot a; target tile a's go to slot b (in
     // a diagonal block both are the same rows, and this thread wrote its
     // row's source sums above)
-    const int64_t i = a * kSymBS + tid;
+    const int64_t i = a * TS + tid;
     if (i < n) {
         const int64_t slot = diag ? a : b;
 #pragma unroll
@@ -681,7 +683,7 @@ __global__ __launch_bounds__(kSymBS) __attribute__((amdgpu_waves_per_eu(COMB ? 3
     }
     s_k[tid] = kb;
     __syncthreads();
-    for (int off = kSymBS / 2; off > 0; off >>= 1) {
+    for (int off = TS / 2; off > 0; off >>= 1) {
         if (tid < off) s_k[tid] += s_k[tid + off];
         __syncthreads();
     }
@@ -698,6 +700,8 @@ __global__ __launch_bounds__(256) void k_adj_sym_reduce(AdjOut o, int64_t S) {
     double R[NR];
 #pragma unroll
     for (int r = 0; r < NR; ++r) R[r] = 0.0;
+    // few blocks: several slots' loads in flight per thread
+#pragma unroll 4
     for (int64_t c = 0; c < S; ++c) {
 #pragma unroll
         for (int r = 0; r < NR; ++r) R[r] += o.partr[(c * NR + r) * o.n + j];
@@ -782,19 +786,23 @@ void pick(int kind, SrcFn &fs, SrcFn &ft) {
 
 using SymAdjFn = void (*)(const AdjSymArgs &, int64_t, hipStream_t);
 
-template <int PDE, int DIM, int KIND>
-void adj_sym_launch(const AdjSymArgs &a, int64_t nblocks, hipStream_t s) {
+template <int PDE, int DIM, int KIND, int TS>
+void adj_sym_tile(const AdjSymArgs &a, dim3 g, hipStream_t s) {
     if constexpr (PDE == INTI_HELMHOLTZ && DIM == 3 && KIND == INTI_COMB_SD) {
         if (a.chik) {
-            if (a.comb)
-                hipLaunchKernelGGL((k_adj_sym<PDE, DIM, KIND, true, true>), dim3((unsigned)nblocks), dim3(kSymBS), 0, s, a);
-            else
-                hipLaunchKernelGGL((k_adj_sym<PDE, DIM, KIND, false, true>), dim3((unsigned)nblocks), dim3(kSymBS), 0, s, a);
+            if (a.comb) hipLaunchKernelGGL((k_adj_sym<PDE, DIM, KIND, true, true, TS>), g, dim3(TS), 0, s, a);
+            else hipLaunchKernelGGL((k_adj_sym<PDE, DIM, KIND, false, true, TS>), g, dim3(TS), 0, s, a);
             return;
         }
     }
-    if (a.comb) hipLaunchKernelGGL((k_adj_sym<PDE, DIM, KIND, true>), dim3((unsigned)nblocks), dim3(kSymBS), 0, s, a);
-    else hipLaunchKernelGGL((k_adj_sym<PDE, DIM, KIND, false>), dim3((unsigned)nblocks), dim3(kSymBS), 0, s, a);
+    if (a.comb) hipLaunchKernelGGL((k_adj_sym<PDE, DIM, KIND, true, false, TS>), g, dim3(TS), 0, s, a);
+    else hipLaunchKernelGGL((k_adj_sym<PDE, DIM, KIND, false, false, TS>), g, dim3(TS), 0, s, a);
+}
+
+template <int PDE, int DIM, int KIND>
+void adj_sym_launch(const AdjSymArgs &a, int64_t nblocks, hipStream_t s) {
+    if (a.tile == kSymBS) adj_sym_tile<PDE, DIM, KIND, kSymBS>(a, dim3((unsigned)nblocks), s);
+    else adj_sym_tile<PDE, DIM, KIND, kAdjSmallTile>(a, dim3((unsigned)nblocks), s);
 }
 
 template <int PDE, int DIM>
@@ -1030,13 +1038,20 @@ int op_adjoint(Op *op, const double *ubar, const double *sigma, double *sigma_ba
     for (int64_t j = 0; j < n; ++j) hs[j] = cplx ? make_double2(sigma[2 * j], sigma[2 * j + 1]) : make_double2(sigma[j], 0.0);
 
     hipStream_t s = ctx->stream;
-    // symmetric pullback: an operator on one quadrature, every output in one
-    // pass over the unordered pairs
     const int NRs = comb ? 2 * dim + 2 : 3 * dim + 2;
-    const int64_t symT = (n + kSymBS - 1) / kSymBS;
+    // symmetric pullback: an operator on one quadrature, every output in one
+    // pass over the unordered pairs. Two-wave tiles of 128 nodes up to 12 blocks
+    // of 256-node tiles per CU (about 20,000 nodes): they fill the last round
+    // better and leave no CU idle (every gradient of the 3D Helmholtz CF, 6,000
+    // nodes: 342 -> 296 us with the call's copies, 17,280: 1068 -> 1033); beyond,
+    // twice the partial slots cost more (30,720: 2790 -> 2872). The symmetric
+    // sum is faster than the two passes from two tiles on (600 nodes 332 -> 209,
+    // 6,000: 617 -> 296, 2D 6,000: 1045 -> 491).
+    const int64_t bigT = (n + kSymBS - 1) / kSymBS;
+    const int tile = bigT * (bigT + 1) / 2 < 12LL * ctx->num_cu ? kAdjSmallTile : kSymBS;
+    const int64_t symT = (n + tile - 1) / tile;
     SymAdjFn fsym = nullptr;
-    const bool sym_fills = op->sym == 2 || symT * (symT + 1) / 2 >= 2LL * ctx->num_cu;
-    if (op->sym && sym_fills && op->trg == op->src && !ff && symT >= 2 &&
+    if (op->sym && op->trg == op->src && !ff && symT >= 2 &&
         sizeof(double) * (size_t)symT * NRs * (size_t)n <= kAdjSymMaxBytes) {
         if (op->pde == INTI_LAPLACE && dim == 2) fsym = pick_sym<INTI_LAPLACE, 2>(kind);
         if (op->pde == INTI_LAPLACE && dim == 3) fsym = pick_sym<INTI_LAPLACE, 3>(kind);
@@ -1093,6 +1108,7 @@ int op_adjoint(Op *op, const double *ubar, const double *sigma, double *sigma_ba
         sa.c = dc; sa.sig = dsg;
         sa.part = dpart; sa.kpart = dkp;
         sa.ntiles = symT;
+        sa.tile = tile;
         sa.distinct = op->src->distinct ? 1 : 0;
         sa.comb = comb ? 1 : 0;
         sa.chik = op->pde == INTI_HELMHOLTZ && dim == 3 && kind == INTI_COMB_SD && p.c1.x == 1.0 && p.c1.y == 0.0 &&
