@@ -481,10 +481,11 @@ int launch_apply(const DirectLaunch &L) {
             ra.split = n > 0 ? nsplit : 0;
             ra.part = part;
             // four waves per 64 rows from 16 partials on, while blocks of 256
-            // rows would leave CUs with fewer than four (a solve of 4,320 nodes
-            // with 68 partials per row: 1,975 -> 1,889 us for 26 sums; one sum of
-            // 6,006: 172 -> 168)
-            const bool few = ra.split >= 16 && ntiles * nr < 4LL * ctx->num_cu;
+            // rows would leave CUs idle (a solve of 4,320 nodes with 68 partials
+            // per row: 1,975 -> 1,889 us for 26 sums; one sum of 6,006: 172 -> 168;
+            // with 480 blocks, 122,880 nodes, it is bound by bandwidth and the
+            // longer rows of the one-thread form are read faster: 95 / 103)
+            const bool few = ra.split >= 16 && ntiles * nr < ctx->num_cu;
             dim3 rg((unsigned)(few ? (m + 63) / 64 : ntiles), (unsigned)nr);
             if (few && cplx) hipLaunchKernelGGL((k_reduce<true, 4>), rg, dim3(256), 0, ctx->stream, ra);
             else if (few) hipLaunchKernelGGL((k_reduce<false, 4>), rg, dim3(256), 0, ctx->stream, ra);
