@@ -245,7 +245,8 @@ static int quad_distinct(const Quad *q) {
         int *dflag = (int *)(box + nbox);
         hipStream_t s = ctx->stream;
         INTI_HIP(ctx, hipMemcpyAsync(dflag, &flag, sizeof(int), hipMemcpyHostToDevice, s));
-        const int64_t pairs = T * (T + 1) / 2, most = int64_t(1) << 24;
+        // a launch holds fewer than 2^32 threads (1,483,008 nodes need more)
+        const int64_t pairs = T * (T + 1) / 2, most = (int64_t(1) << 32) / kSymBS - 1;
         if (q->dim == 2) hipLaunchKernelGGL(k_tile_boxes<2>, dim3((unsigned)T), dim3(kSymBS), 0, s, n, q->coords, box, dflag);
         else hipLaunchKernelGGL(k_tile_boxes<3>, dim3((unsigned)T), dim3(kSymBS), 0, s, n, q->coords, box, dflag);
         for (int64_t f = 0; f < pairs; f += most) {
