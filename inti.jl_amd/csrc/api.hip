@@ -222,6 +222,29 @@ __global__ __launch_bounds__(kSymBS) void k_close_pairs(int64_t n, int64_t T, in
     if (close) *flag = 1;
 }
 
+// Creating an operator must not disturb captures: with the thread's capture
+// mode relaxed, the allocation, the copies and the wait below are allowed while
+// other streams are being captured (in the global mode hipMalloc is refused
+// then and ends their capture). The quadrature's device is made current.
+struct OutsideCaptures {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    int device = 0;
+    bool moved = false;
+    hipError_t err;
+    explicit OutsideCaptures(int dev) {
+        err = hipThreadExchangeStreamCaptureMode(&mode);
+        if (err == hipSuccess) err = hipGetDevice(&device);
+        if (err == hipSuccess && device != dev) {
+            err = hipSetDevice(dev);
+            moved = err == hipSuccess;
+        }
+    }
+    ~OutsideCaptures() {
+        if (moved) (void)hipSetDevice(device);
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
 // Decides q->distinct once, on the stream of the quadrature's context (locked
 // by the caller). While that stream is being captured nothing is launched and
 // the question stays open: the mask is kept, and the next operator asks again.
@@ -231,6 +254,8 @@ static int quad_distinct(const Quad *q) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     INTI_HIP(ctx, hipStreamIsCapturing(ctx->stream, &cap));
     if (cap != hipStreamCaptureStatusNone) return INTI_OK;
+    OutsideCaptures outside(ctx->device);
+    INTI_HIP(ctx, outside.err);
     const int64_t n = q->n, T = (n + kSymBS - 1) / kSymBS;
     int flag = 0;
     if (n > 0) {

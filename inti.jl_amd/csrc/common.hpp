@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <memory>
 #include <mutex>
@@ -49,8 +50,9 @@ struct Quad {
     double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};  // bounding box
     // no two nodes within 2x the coincidence tolerance: pairs of different
     // nodes then never need the coincident-point mask (decided when the first
-    // operator with this quadrature as target and source is created)
-    mutable bool distinct = false, distinct_known = false;
+    // operator with this quadrature as target and source is created, under the
+    // lock of ctx; operators of other contexts read it under their own)
+    mutable std::atomic<bool> distinct{false}, distinct_known{false};
 };
 
 // CSR with 0-based int32 indices; values real (double) or complex

@@ -4,6 +4,8 @@ partial one, a pair closer than the coincidence tolerance apart, and none.
 The symmetric sum drops its coincidence mask only for distinct nodes; with a
 coincident pair left unmasked the sums are infinite or NaN, so the apply is
 compared with the oracle (FP64 <= 1e-12)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -54,3 +56,54 @@ def test_many_nodes(inti):
     y = inti.IntegralOperator(inti.DoubleLayerKernel(inti.Laplace(dim=2)), T, Q) @ np.ones(n)
     print(f"[gpu] {n} nodes: {y}", flush=True)
     assert np.all(np.abs(y + 0.5 - 0.5 / n) <= 1e-9)
+
+
+@pytest.mark.parametrize("captured", ["own stream", "another stream"])
+@pytest.mark.parametrize("pair", [None, (3, 900)])
+def test_operator_made_during_a_capture(inti, oracle, captured, pair):
+    """An operator made while a stream is captured in the global mode (its
+    context's own, where the test is put off, or another): the capture ends
+    whole, its graph replays, and the operator masks a coincident pair."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    n = 1300
+    i = np.arange(n) + 0.5
+    X = np.stack([np.cos(2 * np.pi * i / n), np.sin(2 * np.pi * i / n)])
+    if pair:
+        X[:, pair[1]] = X[:, pair[0]]
+    Q = inti.Quadrature(X, X, np.full(n, 1.0 / n), np.zeros((1, 0), dtype=np.int64))
+    ctx = inti.default_context()
+    Q.device(ctx)
+    own, stream, dev = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    ctx.check(ctx.lib.inti_ctx_stream(ctx.handle, ctypes.byref(own)))
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(stream), 1) == 0
+    s = own if captured == "own stream" else stream
+    src, dst = (ctypes.c_double * 4)(1.0, 2.0, 3.0, 4.0), (ctypes.c_double * 4)()
+    assert hip.hipMalloc(ctypes.byref(dev), ctypes.c_size_t(64)) == 0
+    up = ctypes.c_void_p(dev.value + 32)
+    assert hip.hipMemcpy(dev, src, ctypes.c_size_t(32), 1) == 0
+    graph, run = ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamBeginCapture(s, 0) == 0
+    try:
+        rc = hip.hipMemcpyAsync(up, dev, ctypes.c_size_t(32), 3, s)
+        A = inti.IntegralOperator(inti.SingleLayerKernel(inti.Laplace(dim=2)), Q, Q)
+        A.handle
+    finally:
+        ended = hip.hipStreamEndCapture(s, ctypes.byref(graph))
+    assert rc == 0 and ended == 0
+    assert hip.hipGraphInstantiate(ctypes.byref(run), graph, None, None, ctypes.c_size_t(0)) == 0
+    x = np.random.default_rng(1).normal(size=n)
+    ref = oracle.matvec(0, 2, 0, 0.0, Q, Q, x).real
+    B = inti.IntegralOperator(inti.SingleLayerKernel(inti.Laplace(dim=2)), Q, Q)
+    for r in range(3):
+        src[0] = float(r)
+        assert hip.hipMemcpy(dev, src, ctypes.c_size_t(32), 1) == 0
+        assert hip.hipGraphLaunch(run, s) == 0 and hip.hipStreamSynchronize(s) == 0
+        assert hip.hipMemcpy(dst, up, ctypes.c_size_t(32), 2) == 0
+        assert list(dst) == list(src)
+        for op in (A, B):
+            op.set_symmetric(2)
+            y = op @ x
+            print(f"[gpu] {captured}, pair {pair}: {np.linalg.norm(y - ref) / np.linalg.norm(ref):.2e}", flush=True)
+            assert np.linalg.norm(y - ref) <= 1e-12 * np.linalg.norm(ref)
+    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
+    assert hip.hipFree(dev) == 0 and hip.hipStreamDestroy(stream) == 0
