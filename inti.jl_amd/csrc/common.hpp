@@ -146,9 +146,8 @@ struct DirectLaunch {
     size_t part_bytes = 0;
 };
 int launch_apply(const DirectLaunch &L);
-// allocate the scratch an apply of nrhs columns needs (before graph capture);
-// rows: x and y don't overlap, so the one-launch sum may be taken
-int apply_reserve(const Op *op, int nrhs, bool rows = true);
+// allocate the scratch an apply of nrhs columns needs (before graph capture)
+int apply_reserve(const Op *op, int nrhs);
 int gmres_solve(Op *op, Op *prec, const double *b, double *x, int restart, int maxiter, double rtol,
                 double atol, int use_graph, int *iters, double *relres);
 int refine_solve(Op *op_hi, Op *op_lo, Op *prec, const double *b, double *x, int restart, int maxiter_inner,

@@ -303,7 +303,7 @@ KParams op_params(const Op *op, int *eff_kind) {
 // 4 columns, 3D Helmholtz DL, 4,320 nodes 100 -> 75 us, 9,000: 280 -> 224; 16
 // columns, 1,700 nodes 79 -> 31, 4,320: 115 -> 102.
 constexpr int64_t kChunkCost = 8;
-static void plan_split(const Op *op, int64_t m, int64_t n, ApplyFn fn, int nr, int &split, int64_t &chunk) {
+static int64_t base_split(const Op *op, int64_t m, int64_t n) {
     const int64_t ntiles = (m + kApplyBS - 1) / kApplyBS;
     const int64_t stiles = (n + kApplyBS - 1) / kApplyBS;
     int64_t s0 = op->split;
@@ -311,7 +311,13 @@ static void plan_split(const Op *op, int64_t m, int64_t n, ApplyFn fn, int nr, i
         s0 = (8LL * op->ctx->num_cu + ntiles - 1) / ntiles;
         if (s0 >= 8) s0 = (s0 + 7) / 8 * 8;
     }
-    s0 = std::max<int64_t>(1, std::min(s0, stiles));
+    return std::max<int64_t>(1, std::min(s0, stiles));
+}
+
+static void plan_split(const Op *op, int64_t m, int64_t n, ApplyFn fn, int nr, int &split, int64_t &chunk) {
+    const int64_t ntiles = (m + kApplyBS - 1) / kApplyBS;
+    const int64_t stiles = (n + kApplyBS - 1) / kApplyBS;
+    const int64_t s0 = base_split(op, m, n);
     chunk = (stiles + s0 - 1) / s0 * kApplyBS;
     if (op->split <= 0 && fn && n > 0) {
         const int64_t gran = nr == 16 ? kMfmaTT : nr == 4 ? ApplyTile<4>::TT : ApplyTile<1>::TT;
@@ -333,31 +339,27 @@ static void plan_split(const Op *op, int64_t m, int64_t n, ApplyFn fn, int nr, i
     if (split < 1) split = 1;
 }
 
-// scratch of the column blocks (16, 4, 1) a call of nrhs columns uses
-int apply_reserve(const Op *op, int nrhs, bool rows) {
+// Scratch of the column blocks (16, 4, 1) of a call of nrhs columns, one column
+// among them always and both the symmetric and the one-direction sums, also
+// where the call takes the one-launch sum and needs none: after one eager call,
+// calls of the same operator with one column, with overlapping operands or
+// with set_symmetric(0) allocate nothing, as a stream capture requires.
+int apply_reserve(const Op *op, int nrhs) {
     const int cw = op_is_complex(op) ? 2 : 1;
     const int64_t m = op->trg->n, n = op->src->n;
     int kind = op->kind;
     SymPlan sp;
     (void)op_params(op, &kind);
-    size_t bytes = 0;
-    for (int nr : {16, 4, 1}) {
+    // one column: at most twice the base split (plan_split)
+    size_t bytes = sizeof(double) * cw * (size_t)m * 2 * base_split(op, m, n);
+    for (int nr : {16, 4}) {
         if (nrhs < nr) continue;
-        if (nr == 1) {
-            const bool sym = plan_sym(op, kind, sp);
-            if (rows && plan_row(op, m, n, sym, nr)) continue;
-            if (sym) {
-                bytes = std::max(bytes, sizeof(double) * cw * (size_t)sp.S * (size_t)n);
-                continue;
-            }
-        } else if (rows && plan_row(op, m, n, false, nr)) {
-            continue;
-        }
         int split;
         int64_t chunk;
         plan_split(op, m, n, pick_apply(op_kernel_pde(op), op->dim, kind, op->precision == INTI_MIXED, nr), nr, split, chunk);
         bytes = std::max(bytes, sizeof(double) * cw * (size_t)m * split * nr);
     }
+    if (plan_sym(op, kind, sp)) bytes = std::max(bytes, sizeof(double) * cw * (size_t)sp.S * (size_t)n);
     void *scr = nullptr;
     return ctx_scratch(op->ctx, kScrPartial, bytes, &scr);
 }
@@ -378,7 +380,7 @@ int launch_apply(const DirectLaunch &L) {
     const double *xend = L.x + cw * ((int64_t)(L.nrhs - 1) * L.ldx + n), *yend = L.y + cw * ((int64_t)(L.nrhs - 1) * L.ldy + m);
     const bool rows = L.x >= yend || L.y >= xend;
     if (!given) {
-        int st = apply_reserve(op, L.nrhs, rows);
+        int st = apply_reserve(op, L.nrhs);
         if (st) return st;
         void *scr = nullptr;
         st = ctx_scratch(ctx, kScrPartial, 0, &scr);
