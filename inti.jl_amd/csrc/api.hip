@@ -56,7 +56,7 @@ int Arena::commit() {
     for (const Cut &c : cuts) total += (c.bytes + 255) / 256 * 256;
     void *at = nullptr;
     if (total <= kArenaKeep) {
-        if (int st = ctx_scratch(ctx, kScrTmp, total, &at)) return st;
+        if (int st = ctx_scratch(ctx, kScrArena, total, &at)) return st;
     } else {
         if (hipMalloc(&own, total) != hipSuccess) {
             own = nullptr;
@@ -353,7 +353,7 @@ int inti_ctx_destroy(inti_ctx *ctx) {
     if (!ctx) return INTI_ERR_ARG;
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
-    for (int s = 0; s < 4; ++s)
+    for (int s = 0; s < Ctx::kSlots; ++s)
         if (ctx->scratch[s]) (void)hipFree(ctx->scratch[s]);
     (void)hipEventDestroy(ctx->ev0);
     (void)hipEventDestroy(ctx->ev1);
@@ -799,7 +799,7 @@ int inti_op_attach_correction(inti_op *op, const inti_csr *csr, double coef_re, 
         if (same && csr->nnz > 0) {
             int differ = 0, *dflag = nullptr;
             void *scr = nullptr;
-            if (int st = ctx_scratch(ctx, kScrTmp, sizeof(int), &scr)) return st;
+            if (int st = ctx_scratch(ctx, kScrArena, sizeof(int), &scr)) return st;
             dflag = (int *)scr;
             INTI_HIP(ctx, hipMemcpyAsync(dflag, &differ, sizeof(int), hipMemcpyHostToDevice, ctx->stream));
             hipLaunchKernelGGL(k_differ, dim3((unsigned)((csr->m + 256) / 256)), dim3(256), 0, ctx->stream, csr->m + 1,

@@ -32,9 +32,11 @@ struct Ctx {
     float last_kernel_ms = 0.f;
     int num_cu = 256;
     // scratch slots (grown on demand, freed at destroy): 0 partial sums,
-    // 1-2 staging of host operands, 3 correction-build temporaries
-    void *scratch[4] = {nullptr, nullptr, nullptr, nullptr};
-    size_t scratch_bytes[4] = {0, 0, 0, 0};
+    // 1-2 staging of host operands, 3 dense products, 4 temporaries of
+    // builds, pullbacks and attaches (Arena)
+    static constexpr int kSlots = 5;
+    void *scratch[kSlots] = {};
+    size_t scratch_bytes[kSlots] = {};
     // device address of the library's static partial-sum buffer on this
     // context's device (the allocation-free apply)
     double *noalloc_scratch = nullptr;
@@ -100,13 +102,16 @@ int set_error(Ctx *ctx, int code, const std::string &msg);
     } while (0)
 
 // scratch memory of the context (grown on demand; never shrinks)
-enum { kScrPartial = 0, kScrX = 1, kScrY = 2, kScrTmp = 3 };
+enum { kScrPartial = 0, kScrX = 1, kScrY = 2, kScrTmp = 3, kScrArena = 4 };
 int ctx_scratch(Ctx *ctx, int slot, size_t bytes, void **ptr);
 
 // The device temporaries of one call: sizes are added, then one buffer is cut
 // into them (256-byte aligned). Up to kArenaKeep bytes the buffer is the
-// context's kScrTmp scratch, kept for the next call; beyond, an allocation of
-// this call alone. The arena drains the stream when it goes (an error return
+// context's kScrArena scratch, kept for the next call (growing, it takes a
+// quarter more than asked for: at most 640 MiB, until the context goes);
+// beyond, an allocation of this call alone. The slot is the arena's own: one
+// that captured calls read (kScrPartial, kScrTmp) would leave their graphs
+// with freed memory when a build or a pullback grows it. The arena drains the stream when it goes (an error return
 // may leave copies from the call's host vectors queued: declare those first).
 class Arena {
   public:

@@ -69,3 +69,41 @@ def test_captured_after_one_eager_call(inti, pde, dim, n, eager_cols, in_place, 
         assert err <= 1e-13
     assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
     assert hip.hipFree(dx) == 0 and hip.hipFree(dy) == 0
+
+
+def test_dense_product_outlives_builds(inti):
+    hip, ctx = ctypes.CDLL("libamdhip64.so"), inti.Context(0)
+    CONTEXTS.append(ctx)
+    Q = inti.sphere_quadrature(3, qorder=4)
+    n, nrhs, op = len(Q), 3, inti.Helmholtz(k=2.0, dim=3)
+    S = inti.IntegralOperator(inti.SingleLayerKernel(op), Q, Q, ctx=ctx)
+    D = inti.IntegralOperator(inti.DoubleLayerKernel(op), Q, Q, ctx=ctx)
+    M = inti.DenseOperator(D)
+    rng = np.random.default_rng(3)
+    x = rng.normal(size=(nrhs, n)) + 1j * rng.normal(size=(nrhs, n))
+    ref, y = np.ascontiguousarray(M.apply(x.T).T), np.empty_like(x)
+    one, zero = (ctypes.c_double * 2)(1.0, 0.0), (ctypes.c_double * 2)(0.0, 0.0)
+    dx, dy, graph, run = (ctypes.c_void_p() for _ in range(4))
+    for d in (dx, dy):
+        assert hip.hipMalloc(ctypes.byref(d), ctypes.c_size_t(x.nbytes)) == 0
+    assert hip.hipMemcpy(dx, x.ctypes.data_as(ctypes.c_void_p), ctypes.c_size_t(x.nbytes), 1) == 0
+    s = ctypes.c_void_p(ctx.stream())
+    assert hip.hipStreamBeginCapture(s, 1) == 0
+    rc = ctx.lib.inti_dense_gemm(ctx.handle, 1, n, n, nrhs, M.device_pointer, n, dx, n, dy, n, one, zero)
+    assert hip.hipStreamEndCapture(s, ctypes.byref(graph)) == 0
+    ctx.check(rc)
+    assert hip.hipGraphInstantiate(ctypes.byref(run), graph, None, None, ctypes.c_size_t(0)) == 0
+    for r in range(3):
+        dS, dD = inti.bdim_correction(op, Q, Q, S, D, green_multiplier=np.full(n, -0.5))
+        E = inti.IntegralOperator(inti.DoubleLayerKernel(op), Q, Q, ctx=ctx)
+        E.attach(dD)
+        E.attach(dS, 0.3)
+        E.pullback(x[0], x[1])
+        assert hip.hipMemcpy(dy, x.ctypes.data_as(ctypes.c_void_p), ctypes.c_size_t(x.nbytes), 1) == 0
+        assert hip.hipGraphLaunch(run, s) == 0
+        ctx.synchronize()
+        assert hip.hipMemcpy(y.ctypes.data_as(ctypes.c_void_p), dy, ctypes.c_size_t(x.nbytes), 2) == 0
+        print(f"[gpu] dense product, replay {r}: {np.linalg.norm(y - ref) / np.linalg.norm(ref):.2e}", flush=True)
+        assert np.array_equal(y, ref)
+    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
+    assert hip.hipFree(dx) == 0 and hip.hipFree(dy) == 0
