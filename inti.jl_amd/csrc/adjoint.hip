@@ -1081,6 +1081,10 @@ int op_adjoint(Op *op, const double *ubar, const double *sigma, double *sigma_ba
     const size_t part_bytes = fsym ? sizeof(double) * (size_t)symT * NRs * (size_t)n
                                    : std::max(sizeof(double2) * (size_t)split_s * n * NVs,
                                               xbar ? sizeof(double2) * (size_t)split_t * m * dim : 0);
+    // host ends of the copies below, which the arena drains. Combined node
+    // gradient: the symmetric pass sums the two parts, the two-pass path adds
+    // the target part on the host
+    std::vector<double> kp(nsb), xsep(comb && !fsym ? (size_t)dim * m : 0);
     if (sigma_bar)
         if (int rc = op_transpose_correction(op)) return rc;
     double2 *dc, *dsg;
@@ -1171,14 +1175,10 @@ int op_adjoint(Op *op, const double *ubar, const double *sigma, double *sigma_ba
                            dsb);
         INTI_HIP(ctx, hipGetLastError());
     }
-    std::vector<double> kp(nsb);
     if (sigma_bar) INTI_HIP(ctx, hipMemcpyAsync(sigma_bar, dsb, sizeof(double) * (cplx ? 2 : 1) * n, hipMemcpyDeviceToHost, s));
     if (ybar) INTI_HIP(ctx, hipMemcpyAsync(ybar, dyb, sizeof(double) * dim * n, hipMemcpyDeviceToHost, s));
     if (nbar) INTI_HIP(ctx, hipMemcpyAsync(nbar, dnb, sizeof(double) * dim * n, hipMemcpyDeviceToHost, s));
     if (wbar) INTI_HIP(ctx, hipMemcpyAsync(wbar, dwb, sizeof(double) * n, hipMemcpyDeviceToHost, s));
-    // combined node gradient: the symmetric pass summed the two parts; the
-    // two-pass path adds the target part on the host
-    std::vector<double> xsep(comb && !fsym ? (size_t)dim * m : 0);
     if (xbar && !(comb && fsym))
         INTI_HIP(ctx, hipMemcpyAsync(comb ? xsep.data() : xbar, dxb, sizeof(double) * dim * m, hipMemcpyDeviceToHost, s));
     if (kbar) INTI_HIP(ctx, hipMemcpyAsync(kp.data(), dkp, sizeof(double) * nsb, hipMemcpyDeviceToHost, s));

@@ -621,7 +621,8 @@ int bdim_build_types(Op *opS, Op *opD, int deriv, int ntypes, const int *nq, con
     int32_t *dqt, *dglob, *dpp, *dploc, *delems, *dseg, *dperm;
     double2 *dB0, *dB1, *dpart, *dth, *dtriS, *dtriD;
     const size_t cb = sizeof(double2), ib = sizeof(int32_t);
-    TripletPattern pat;  // outlives the arena, which drains the uploads
+    TripletPattern pat;  // these two outlive the arena, which drains the copies
+    std::vector<double> dg(3 * elems.size());
     Arena mem(ctx);
     mem.add(&dzs, zs.size() * sizeof(double));
     mem.add(&dqt, qt32.size() * ib);
@@ -763,7 +764,6 @@ int bdim_build_types(Op *opS, Op *opD, int deriv, int ntypes, const int *nq, con
         launch_gather1(g, st);
         if (hipGetLastError() != hipSuccess) return fail(set_error(ctx, INTI_ERR_HIP, "bdim: gather launch failed"));
     }
-    std::vector<double> dg(3 * elems.size());
     if (!dg.empty() &&
         hipMemcpyAsync(dg.data(), ddiag, sizeof(double) * dg.size(), hipMemcpyDeviceToHost, st) != hipSuccess)
         return fail(set_error(ctx, INTI_ERR_HIP, "bdim: diag copy failed"));
