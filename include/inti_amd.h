@@ -133,7 +133,10 @@ int inti_op_set_identity(inti_op *op, double re, double im);
  * operator. */
 int inti_op_set_wavenumber_imag(inti_op *op, double kimag);
 /* Launch shape: threads per block, targets per thread, source splits
- * (0 = automatic). Used by the tuner; defaults are sensible. */
+ * (0 = automatic). Used by the tuner; defaults are sensible. The splits are
+ * the one-direction sum's; with a split given, a square operator takes the
+ * symmetric sum in automatic mode only where 256-node tiles give every CU two
+ * blocks (about 8,000 nodes on MI355X). */
 int inti_op_set_launch(inti_op *op, int block, int tpt, int split);
 /* Symmetric evaluation of a square operator whose target and source are the
  * same quadrature handle (single right-hand side): each unordered pair's

@@ -183,6 +183,9 @@ bool plan_sym(const Op *op, int kind, SymPlan &P) {
     const int64_t n = op->src->n;
     auto tiles = [n](int tile) { return (n + tile - 1) / tile; };
     if (tiles(kSymBS) < 2) return false;
+    // a source split asked for (inti_op_set_launch) is the one-direction sum's:
+    // automatic mode keeps that sum where 256-node tiles leave CUs idle
+    if (op->sym == 1 && op->split > 0 && tiles(kSymBS) * (tiles(kSymBS) + 1) / 2 < 2LL * op->ctx->num_cu) return false;
     const size_t es = sizeof(double) * (op_is_complex(op) ? 2 : 1);
     if (op->sym_group == 0) {
         const int64_t t128 = tiles(128), t256 = tiles(kSymBS), cu = op->ctx->num_cu;
