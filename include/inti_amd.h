@@ -144,8 +144,9 @@ int inti_op_set_launch(inti_op *op, int block, int tpt, int split);
  * in both directions. mode 0: off; 1 (default): where it is the faster sum
  * (from about 1,800 nodes, 3,400 for 2D Helmholtz); 2: wherever it applies
  * (more than 256 nodes). group: tiles of 256 nodes per work group (1, 2 or
- * 4); 0: automatic, tiles of 64 or 128 nodes for smaller sums, else the
- * smallest group whose partial sums fit 4 GiB. Results are
+ * 4; in mode 1 from about 8,000 nodes on, one direction below); 0: automatic,
+ * tiles of 64 or 128 nodes for smaller sums, else the smallest group whose
+ * partial sums fit 4 GiB. Results are
  * deterministic in every mode. No counterpart in Inti.jl (its matrices are
  * assembled entry by entry). */
 int inti_op_set_symmetric(inti_op *op, int mode, int group);

@@ -176,16 +176,21 @@ constexpr size_t kSymSmallBytes = size_t(512) << 20;
 //   2D Helmholtz CF FP64   6,006: 333 / - / 179 (328)  30,720: 2592 / - / 2583
 //   2D Helmholtz CF mixed  6,006: 123 / - / 82 (146)   40,000: 1989 / - / 2019
 // Sums of 256 nodes or fewer run in one direction (k_apply_row). An explicit
-// group keeps tiles of 256. Beyond kSymMaxBytes of partial sums the groups of
+// group has tiles of 256. Beyond kSymMaxBytes of partial sums the groups of
 // 2 and 4 tiles halve and quarter them.
 bool plan_sym(const Op *op, int kind, SymPlan &P) {
     if (op->sym == 0 || op->trg != op->src || kind >= INTI_FF_SL || op->kimag != 0.0) return false;
     const int64_t n = op->src->n;
     auto tiles = [n](int tile) { return (n + tile - 1) / tile; };
     if (tiles(kSymBS) < 2) return false;
-    // a source split asked for (inti_op_set_launch) is the one-direction sum's:
-    // automatic mode keeps that sum where 256-node tiles leave CUs idle
-    if (op->sym == 1 && op->split > 0 && tiles(kSymBS) * (tiles(kSymBS) + 1) / 2 < 2LL * op->ctx->num_cu) return false;
+    // a source split asked for (inti_op_set_launch) is the one-direction sum's,
+    // and a group asked for is one of 256-node tiles: automatic mode takes those
+    // two where the tile pairs give every CU two blocks. Below, one direction is
+    // faster than such groups (4,320 nodes with groups of 1 / 4: 3D Helmholtz CF
+    // 101 / 1,522 us against 85, mixed 3D Laplace SL 41 / 519 against 24)
+    if (op->sym == 1 && (op->split > 0 || op->sym_group > 0) &&
+        tiles(kSymBS) * (tiles(kSymBS) + 1) / 2 < 2LL * op->ctx->num_cu)
+        return false;
     const size_t es = sizeof(double) * (op_is_complex(op) ? 2 : 1);
     if (op->sym_group == 0) {
         const int64_t t128 = tiles(128), t256 = tiles(kSymBS), cu = op->ctx->num_cu;

@@ -162,3 +162,17 @@ def test_explicit_split(inti, pde, dim, kind, n):
     err = np.linalg.norm(out[1, 1] - out[1, 2]) / np.linalg.norm(out[1, 1])
     say(f"[gpu] explicit split pde {pde} dim {dim} n={n}: 1 / 2 chunks differ by {err:.1e}")
     assert 0 < err <= 1e-13
+
+
+# an explicit group in automatic mode: below two blocks of 256-node tile pairs
+# per CU the sum without the symmetric one, above it the group's own, bit for bit
+@pytest.mark.parametrize("pde,dim,kind,precision", [(0, 3, 0, "mixed"), (1, 3, 4, "fp64"), (1, 2, 1, "fp64")])
+@pytest.mark.parametrize("n", [300, 4320, 7900, 9000])
+@pytest.mark.parametrize("group", [1, 2, 4])
+def test_explicit_group(inti, pde, dim, kind, precision, n, group):
+    Q = _nodes(inti, dim, n)
+    x = np.random.default_rng(5).normal(size=n) + (1j if pde else 0.0)
+    A, B = (inti.IntegralOperator(_kernel(inti, pde, dim, kind)[0], Q, Q, precision=precision) for _ in range(2))
+    A.set_symmetric(1, group)
+    B.set_symmetric(2 if n == 9000 else 0, group)
+    assert np.array_equal(A @ x, B @ x)
