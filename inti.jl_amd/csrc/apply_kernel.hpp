@@ -478,28 +478,34 @@ __device__ __forceinline__ void reduce_epilogue(const ReduceArgs &a, int64_t i, 
 }
 
 // ------------------------------------------------------ small sums, one launch
-// NR (1 or 4) right-hand sides of few targets in one launch: a block takes tb
-// targets (4 ... 64, a power of two) and 256 / tb threads share each target's
-// sources, thread t of a target taking sources t, t + 256 / tb, ... read
-// straight from memory (consecutive threads read consecutive sources). The
-// threads' sums are added in a fixed order (lanes by a butterfly, then the
-// four waves in wave order) and the block finishes its rows itself (post
-// factor, correction, identity, alpha / beta): no partial sums and no second
-// kernel. See launch_apply for where it is taken.
+// NR (1 or 4) right-hand sides of few targets in one launch: a block takes
+// kRowTargets targets and 64 threads share each target's sources, thread t of a
+// target taking sources t, t + 64, ... read straight from memory (consecutive
+// threads of a target read consecutive sources). The threads' sums are added in
+// a fixed order (lanes by a butterfly, then the four waves in wave order) and
+// the block finishes its rows itself (post factor, correction, identity, alpha /
+// beta): no partial sums and no second kernel. See plan_row for where it is
+// taken.
+constexpr int kRowTargets = 4;
+
 struct RowArgs {
     ApplyArgs s;
     ReduceArgs e;
-    int tb;
+    int tb;  // kRowTargets
 };
 
 template <int PDE, int DIM, int KIND, bool MIXED, int NR>
 __global__ __launch_bounds__(kApplyBS) void k_apply_row(RowArgs a) {
     constexpr bool CPLX = PDE != INTI_LAPLACE;
     constexpr int NW = kApplyBS / 64;
+    // One column: constant strides (3D Helmholtz CF, 3,000 sources 23.9 -> 15.0
+    // us, Laplace DL 16.4 -> 13.1). Four: from the arguments; the schedules of
+    // the constant form were slower (3D Laplace SL, 3,000 sources 13.4 -> 17.5,
+    // 3D Helmholtz DL 23.2 -> 27.4 us)
+    const int tb = NR == 1 ? kRowTargets : a.tb, nsl = kApplyBS / tb;
     __shared__ double2 s_w[NW][NR][64];
     const ApplyArgs &g = a.s;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int tb = a.tb, t = tid & (tb - 1), nsl = kApplyBS / tb;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, t = tid & (tb - 1);
     const int64_t i = (int64_t)blockIdx.x * tb + t;
     const int64_t ic = i < g.m ? i : g.m - 1;
     double xt[DIM], nt[DIM];

@@ -216,39 +216,80 @@ bool plan_sym(const Op *op, int kind, SymPlan &P) {
     return false;
 }
 
-// Targets per block of the one-launch sum (k_apply_row) for nr right-hand
-// sides of m targets and n sources, 0 where another sum is taken.
-// Four targets per block and 64 threads per target keep every thread's
-// source chain short; it reads each source's data once per 16 threads instead
-// of staging it, so it pays where launches, barriers and an idle chip cost
-// more than the loads: few pairs. Against the symmetric sum it is faster up
-// to about 1,800 nodes (3D Helmholtz CF 1,280: 15 / 20 us, 3,000: 41 / 33;
-// 3D Laplace SL 1,280: 8 / 11, 3,000: 23 / 15) and, for 2D Helmholtz, up to
-// 3,400 (CF 3,000: 73 / 102; 4,320: 145 / 125); against the one-direction sum
-// with its second kernel up to 2,400 (Laplace 2,000: 11 / 20; 3,000: 23 / 21)
-// and 3,800 nodes (3D Helmholtz CF 3,000: 40 / 59; 4,320: 85 / 83). The 2D
-// Helmholtz kernels keep it at any size once 4 m threads per CU are in
-// flight: a wave of 4 targets x 16 neighbouring sources takes the same side
-// of the Hankel functions' branch more often than one of 64 targets (CF FP64
-// 12,000: 1264 / 1337 us, 30,720: 7785 / 8235). The chain of a thread is
-// bounded (n <= 8,192) where the targets alone do not fill the chip.
+// Whether nr right-hand sides of m targets and n sources take the one-launch
+// sum (k_apply_row). Four targets per block and 64 threads per target keep
+// every thread's source chain short; it reads each source's data once per 16
+// threads instead of staging it, so it pays where launches, barriers and an
+// idle chip cost more than the loads: few pairs. Against the symmetric sum it
+// is faster up to about 1,800 nodes (3D Helmholtz CF 1,280: 15 / 20 us, 3,000:
+// 41 / 33; 3D Laplace SL 1,280: 8 / 11, 3,000: 23 / 15) and, for 2D Helmholtz,
+// up to 3,400 (CF 3,000: 73 / 102; 4,320: 145 / 125).
+//
+// Against the one-direction sum its time follows the blocks of the fullest CU x
+// the chain of a thread, `work`, at about 0.2 us per unit in 3D Laplace and 0.4
+// in FP64 2D Helmholtz, while the other sum takes 20 - 120 us whatever the size
+// until it fills the chip. So the lines stand at a number of units per kind of
+// pair. One column, m x n (units): times the row form is faster,
+//   Laplace DL, CF         2,040^2 (64): 1.3 - 1.5, 5,000 x 1,000 (80): 1.1 - 1.25,
+//                          2,300^2 (108): 0.83 - 1.0
+//   Laplace SL, HS         2,300^2: 1.04 - 1.2, 300 x 8,192 (128): 0.8 - 1.0; FP64
+//                          logarithms 5,000 x 2,500 (200): 1.3 - 1.6
+//   3D Helmholtz FP64      3,300^2 (208): 1.02 - 1.3, 3,900^2 (244): DL, HS 0.9, SL, CF
+//                          1.0 - 1.1
+//   3D Helmholtz mixed     2,300^2: 1.08 - 1.15, 2,700^2 (129): 0.96 - 1.04; SL, HS
+//                          3,000^2 (141): 1.2, 3,300^2: 0.85 - 0.9
+//   2D far fields          (no Hankel function) FP64 3,900^2: 1.07 - 1.3, 40,000 x
+//                          6,000 (3,760): 0.6 - 0.7; mixed SL 3,600^2 (228): 1.16, CF
+//                          10,000 x 1,000 (160): 1.14, 3,300^2: 0.9, 40,000 x 6,000: 0.3
+//   2D Helmholtz FP64      a wave of 4 targets x 16 neighbouring sources takes the
+//                          same side of the Hankel functions' branch more often than
+//                          one of 64 targets: 40,401 x 2,500 (1,600): 1.06 - 1.13,
+//                          20,000^2 (6,260): 1.08 - 1.13, 30,720^2 (14,400): 0.90 - 1.03
+//   2D Helmholtz mixed     40,401 x 1,000 (640): 1.01 - 1.26, 6,500^2 (714): 0.93 (DL),
+//                          9,000^2: 0.74 - 1.04; 1,024 x 50,000: 0.5 - 0.66
+// With 64 sources or fewer a part of each wave idles, but both sums then grow
+// with m alone: 160,000 x 64: Laplace 0.8 - 1.05, 3D Helmholtz 1.1 - 2.4; 1,000,000
+// x 3: 1.0 - 3, mixed far fields 0.78 - 1.1.
 // Four right-hand sides reuse each pair value, so the staged kernel overtakes
-// earlier: 2,200 nodes in 3D Helmholtz (DL 640: 8 / 36 us, 2,000: 27 / 37,
-// 2,600: 46 / 39), 1,800 for Laplace (3D SL 1,280: 12 / 18, 2,000: 18 / 18)
-// and 3,700 in 2D Helmholtz (CF FP64 1,280: 26 / 140, 3,200: 106 / 156, mixed
-// 3,200: 62 / 72, 4,320: 104 / 90). 16 go to the matrix-core kernel at once.
-static int plan_row(const Op *op, int64_t m, int64_t n, bool sym, int nr) {
-    if (op->split > 0 || n <= 0 || nr > 4) return 0;
+// earlier: 2,048 nodes in 3D Helmholtz (2,040: 1.3 - 1.4x faster, 2,300: 0.8 -
+// 1.05x), 1,800 for Laplace (3D SL 1,280: 12 / 18, 2,000: 18 / 18) and 3,700 in
+// 2D Helmholtz (CF FP64 1,280: 26 / 140, 3,200: 106 / 156, mixed 3,200: 62 / 72,
+// 4,320: 104 / 90); long chains (300 x 4,096 Laplace: 0.8 - 1.1x, 300 x 8,192 3D
+// Helmholtz 0.6x, mixed 2D Helmholtz 0.8x) and many targets of few sources
+// (40,000 x 64 Laplace 0.8 - 1.1x, with FP64 logarithms 1.45x, 200,000 x 4: 82 /
+// 38, 80,000 x 3 mixed 2D Helmholtz 0.9x) are slower. 16 go to the matrix-core kernel at once.
+static bool plan_row(const Op *op, int64_t m, int64_t n, bool sym, int nr) {
+    if (op->split > 0 || n <= 0 || nr > 4) return false;
+    const int kd = op->kind;
+    const bool lap = op->pde == INTI_LAPLACE, ff = kd >= INTI_FF_SL, mixed = op->precision == INTI_MIXED;
+    const bool hankel = !lap && op->dim == 2 && !ff;
+    const bool log64 = lap && op->dim == 2 && !mixed && (kd == INTI_SL || kd == INTI_COMB_SD);
+    const bool dl = kd == INTI_DL || kd == INTI_ADL || (kd == INTI_COMB_SD && !log64);
     const double pairs = (double)m * (double)n;
-    const bool lap = op->pde == INTI_LAPLACE, helm2 = op->pde == INTI_HELMHOLTZ && op->dim == 2;
+    const int64_t span = (int64_t)kRowTargets * op->ctx->num_cu, per_cu = (m + span - 1) / span;
+    double lim;
+    int64_t most_n, most_m;
     if (nr == 4) {
-        const double lim4 = helm2 ? 3700.0 : lap ? 1800.0 : 2200.0;
-        return n <= 8192 && pairs <= lim4 * lim4 ? 4 : 0;
+        if (hankel) lim = 3700.0, most_n = mixed ? 6144 : 8192, most_m = mixed ? 48 : 160;
+        else if (lap) lim = 1800.0, most_n = log64 ? 4096 : 3072, most_m = log64 ? 80 : 20;
+        else if (ff && op->dim == 2 && !mixed) lim = kd == INTI_FF_SL ? 3000.0 : 2240.0, most_n = kd == INTI_FF_SL ? 6144 : 4096, most_m = 20;
+        else if (ff) lim = 2048.0, most_n = mixed ? 3072 : 4096, most_m = 20;
+        else lim = 2048.0, most_n = mixed && dl ? 5120 : 4096, most_m = dl ? 40 : 20;
+        return pairs <= lim * lim && n <= most_n && per_cu <= most_m;
     }
-    if (sym && op->sym == 2) return 0;
-    if (helm2 && !sym && m >= 4LL * op->ctx->num_cu) return 4;
-    const double lim = sym ? (helm2 ? 3400.0 : 1800.0) : (helm2 ? 3400.0 : lap ? 2400.0 : 3800.0);
-    return n <= 8192 && pairs <= lim * lim ? 4 : 0;
+    if (sym) {
+        lim = hankel ? 3400.0 : 1800.0;
+        return op->sym != 2 && pairs <= lim * lim;
+    }
+    const double thin = ff && mixed ? 0.25 : 0.08;  // units of a chain of 16 sources or fewer
+    const double chain = n > 64 ? (double)((n + 63) / 64) : n > 16 ? thin + (0.7 - thin) * (double)(n - 16) / 48.0 : thin;
+    if (hankel) lim = mixed ? 700.0 : 8000.0;
+    else if (lap) lim = log64 ? 200.0 : dl ? 80.0 : 109.0;
+    else if (ff && op->dim == 2) lim = kd == INTI_FF_SL ? 240.0 : mixed ? 190.0 : 250.0;
+    else if (mixed) lim = ff ? 109.0 : dl ? 120.0 : 160.0;
+    else lim = kd == INTI_SL || kd == INTI_COMB_SD || kd == INTI_FF_SL ? 245.0 : 208.0;
+    most_n = hankel && !mixed && m >= span ? INT64_MAX : 8192;
+    return (double)per_cu * chain <= lim && n <= most_n;
 }
 
 KParams op_params(const Op *op, int *eff_kind) {
@@ -417,8 +458,8 @@ int launch_apply(const DirectLaunch &L) {
         ra.cr = op->cid[0]; ra.ci = op->cid[1];
         ra.pr = kp.postr; ra.pi = kp.posti;
         ra.has_id = (op->cid[0] != 0.0 || op->cid[1] != 0.0);
-        const int tb = rows ? plan_row(op, m, n, sym, nr) : 0;
-        RowFn rfn = tb ? pick_row(op_kernel_pde(op), op->dim, kind, op->precision == INTI_MIXED, nr) : nullptr;
+        RowFn rfn = rows && plan_row(op, m, n, sym, nr) ? pick_row(op_kernel_pde(op), op->dim, kind, op->precision == INTI_MIXED, nr)
+                                                           : nullptr;
         ApplyFn fn = rfn || (sym && nr == 1) ? nullptr : pick_apply(op_kernel_pde(op), op->dim, kind, op->precision == INTI_MIXED, nr);
         int split = 1;
         int64_t chunk = n;
@@ -446,9 +487,9 @@ int launch_apply(const DirectLaunch &L) {
             a.s.x = xr; a.s.ldx = L.ldx; a.s.part = nullptr; a.s.split = 0; a.s.chunk = 0;
             a.s.p = kp;
             a.e = ra;
-            a.tb = tb;
+            a.tb = kRowTargets;
             if (ctx->profiling) INTI_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
-            rfn(a, dim3((unsigned)((m + tb - 1) / tb)), ctx->stream);
+            rfn(a, dim3((unsigned)((m + kRowTargets - 1) / kRowTargets)), ctx->stream);
             INTI_HIP(ctx, hipGetLastError());
             if (ctx->profiling) INTI_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
         } else if (n > 0 && nr == 1 && sym) {

@@ -176,3 +176,30 @@ def test_explicit_group(inti, pde, dim, kind, precision, n, group):
     A.set_symmetric(1, group)
     B.set_symmetric(2 if n == 9000 else 0, group)
     assert np.array_equal(A @ x, B @ x)
+
+
+# both sides of the lines between the one-launch sum and the one-direction one
+# (long chains, many targets of few sources, far fields), against the
+# one-direction sum in chunks of its own: the same terms in another order
+@pytest.mark.parametrize("pde,dim,kind", [(0, 2, "SL"), (0, 3, "DL"), (1, 2, "CF"), (1, 3, "SL"), (1, 2, "FFSL"),
+                                          (1, 2, "FFCF"), (1, 3, "FFDL")])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("m,n", [(3, 3657), (3, 6145), (300, 8193), (1023, 16400), (1024, 8200), (2050, 3100), (20480, 64),
+                                 (20481, 65), (180001, 5), (1000003, 3)])
+@pytest.mark.parametrize("nrhs", [1, 4])
+def test_row_lines(inti, pde, dim, kind, precision, m, n, nrhs):
+    Q, T = _nodes(inti, dim, n), _nodes(inti, dim, m, seed=1)
+    T = inti.points(T.coords / np.linalg.norm(T.coords, axis=0) if "FF" in kind else 1.7 * T.coords)
+    op = inti.Helmholtz(k=7.3, dim=dim) if pde else inti.Laplace(dim=dim)
+    K = (inti.CombinedFieldKernel(op, -7.3j, 1.0, "FF" if "FF" in kind else "SD") if "CF" in kind else
+         {"SL": inti.SingleLayerKernel, "DL": inti.DoubleLayerKernel, "FFSL": inti.FarFieldSingleLayerKernel,
+          "FFDL": inti.FarFieldDoubleLayerKernel}[kind](op))
+    rng = np.random.default_rng(17)
+    x = rng.normal(size=(n, nrhs)) + (1j * rng.normal(size=(n, nrhs)) if pde else 0.0)
+    A = inti.IntegralOperator(K, T, Q, precision=precision)
+    y = A @ x
+    A.ctx.check(A.ctx.lib.inti_op_set_launch(A.handle, 256, 1, 3))
+    ref = A @ x
+    err, size = np.linalg.norm(y - ref), np.linalg.norm(ref)
+    say(f"[gpu] {pde} {dim} {kind} {precision} {m} x {n}, {nrhs} columns: {err:.2e} of {size:.2e}")
+    assert err <= (1e-13 if precision == "fp64" else 1e-6) * size
