@@ -257,7 +257,8 @@ bool plan_sym(const Op *op, int kind, SymPlan &P) {
 // 4,320: 104 / 90); long chains (300 x 4,096 Laplace: 0.8 - 1.1x, 300 x 8,192 3D
 // Helmholtz 0.6x, mixed 2D Helmholtz 0.8x) and many targets of few sources
 // (40,000 x 64 Laplace 0.8 - 1.1x, with FP64 logarithms 1.45x, 200,000 x 4: 82 /
-// 38, 80,000 x 3 mixed 2D Helmholtz 0.9x) are slower. 16 go to the matrix-core kernel at once.
+// 38, 80,000 x 3 mixed 2D Helmholtz 0.9x) are slower. 16 go to the matrix-core kernel
+// at once.
 static bool plan_row(const Op *op, int64_t m, int64_t n, bool sym, int nr) {
     if (op->split > 0 || n <= 0 || nr > 4) return false;
     const int kd = op->kind;
@@ -289,7 +290,8 @@ static bool plan_row(const Op *op, int64_t m, int64_t n, bool sym, int nr) {
     else if (mixed) lim = ff ? 109.0 : dl ? 120.0 : 160.0;
     else lim = kd == INTI_SL || kd == INTI_COMB_SD || kd == INTI_FF_SL ? 245.0 : 208.0;
     most_n = hankel && !mixed && m >= span ? INT64_MAX : 8192;
-    return (double)per_cu * chain <= lim && n <= most_n;
+    // (a launch holds fewer than 2^32 threads, 64 per target)
+    return (double)per_cu * chain <= lim && n <= most_n && m < int64_t(1) << 26;
 }
 
 KParams op_params(const Op *op, int *eff_kind) {

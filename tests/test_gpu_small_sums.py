@@ -203,3 +203,19 @@ def test_row_lines(inti, pde, dim, kind, precision, m, n, nrhs):
     err, size = np.linalg.norm(y - ref), np.linalg.norm(ref)
     say(f"[gpu] {pde} {dim} {kind} {precision} {m} x {n}, {nrhs} columns: {err:.2e} of {size:.2e}")
     assert err <= (1e-13 if precision == "fp64" else 1e-6) * size
+
+
+def test_more_targets_than_a_launch_of_64_threads_each(inti):
+    """2^26 targets of three 2D Helmholtz sources (64 threads per target would
+    be 2^32): accepted, and its first, middle and last rows those of a small sum
+    (1e-13, the same pairs by the other kernel)."""
+    m, Q = 1 << 26, _nodes(inti, 2, 3)
+    X = np.empty((2, m))
+    X[0], X[1] = np.linspace(2.0, 9.0, m), 0.5
+    K = inti.SingleLayerKernel(inti.Helmholtz(k=1.3, dim=2))
+    x = np.array([1.0, -0.5j, 0.25 + 1j])
+    rows = np.r_[0:5, m // 2:m // 2 + 5, m - 5:m]
+    y = inti.IntegralOperator(K, inti.points(X), Q).apply(x)[rows]
+    ref = inti.IntegralOperator(K, inti.points(np.ascontiguousarray(X[:, rows])), Q) @ x
+    say(f"[gpu] {m} targets: {np.linalg.norm(y - ref) / np.linalg.norm(ref):.2e}")
+    assert np.linalg.norm(y - ref) <= 1e-13 * np.linalg.norm(ref)
