@@ -347,13 +347,27 @@ KParams op_params(const Op *op, int *eff_kind) {
 // follows the blocks of the fullest CU x chunk whatever the occupancy, and all
 // splits from half to four times the base are looked at, down to one LDS tile
 // (128 or 64 sources) per chunk; a shorter chunk would cost as much as a whole
-// one (the inner loop runs over padding). kChunkCost, in sources, stands for a
+// one (the inner loop runs over padding). chunk_cost, in sources, stands for a
 // block's start and its partial sums; where a lone block per CU waits on its
-// own chains (4 columns, and the 2D Helmholtz kernels) it costs as much as a
-// second one beside it. Against rounds of resident blocks:
-// 4 columns, 3D Helmholtz DL, 4,320 nodes 100 -> 75 us, 9,000: 280 -> 224; 16
-// columns, 1,700 nodes 79 -> 31, 4,320: 115 -> 102.
-constexpr int64_t kChunkCost = 8;
+// own chains (4 columns, and the Hankel functions) it costs as much as a second
+// one beside it. Against rounds of resident blocks: 4 columns, 3D Helmholtz DL,
+// 4,320 nodes 100 -> 75 us, 9,000: 280 -> 224; 16 columns, 1,700 nodes 79 -> 31,
+// 4,320: 115 -> 102.
+// With 16 columns the partial sums weigh more beside cheap pairs. A cost of 8 /
+// 24, us: mixed 2D Helmholtz SL 10,000 nodes 366 / 289, 16,000: 772 / 692; mixed
+// 3D Helmholtz SL 200,000 x 300: 201 / 165, 20,000 x 1,000: 70 / 62; 3D Laplace
+// 200,000 x 300 mixed 99 / 76, FP64 118 / 106; mixed 2D far field 200,000 x 300
+// (with the lone block's cost) 180, without 125. Where the pairs are dear, 24 is
+// too much: FP64 2D Helmholtz SL, 6,500 nodes 8 % slower, FP64 2D Laplace SL
+// 20,000 x 1,000: 60 / 73, FP64 3D Helmholtz CF 102 / 118. The mixed 2D
+// Helmholtz SL and DL take 32 (6,500 nodes 152 / 147).
+static int64_t chunk_cost(const Op *op, int nr) {
+    if (nr != 16) return nr == 1 ? 0 : 8;
+    const int kd = op->kind;
+    if (op->precision == INTI_MIXED)
+        return op->pde == INTI_HELMHOLTZ && op->dim == 2 && (kd == INTI_SL || kd == INTI_DL || kd == INTI_ADL) ? 32 : 24;
+    return op->pde == INTI_LAPLACE && (op->dim == 3 || (kd != INTI_SL && kd != INTI_COMB_SD)) ? 24 : 8;
+}
 static int64_t base_split(const Op *op, int64_t m, int64_t n) {
     const int64_t ntiles = (m + kApplyBS - 1) / kApplyBS;
     const int64_t stiles = (n + kApplyBS - 1) / kApplyBS;
@@ -374,8 +388,9 @@ static void plan_split(const Op *op, int64_t m, int64_t n, ApplyFn fn, int nr, i
         const int64_t gran = nr == 16 ? kMfmaTT : nr == 4 ? ApplyTile<4>::TT : ApplyTile<1>::TT;
         const int64_t gtiles = (n + gran - 1) / gran;
         const int64_t cus = op->ctx->num_cu, cap = nr == 1 ? (int64_t)fn(nullptr, dim3(0), nullptr) * cus : cus;
-        const int64_t lone = nr == 4 || (nr == 16 && op->pde == INTI_HELMHOLTZ && op->dim == 2) ? 1 : 0;
-        const int64_t over = nr == 1 ? 0 : kChunkCost, smax = std::min((nr == 1 ? 2 : 4) * s0, gtiles);
+        const bool hankel = op->pde == INTI_HELMHOLTZ && op->dim == 2 && op->kind < INTI_FF_SL;
+        const int64_t lone = nr == 4 || (nr == 16 && hankel) ? 1 : 0;
+        const int64_t over = chunk_cost(op, nr), smax = std::min((nr == 1 ? 2 : 4) * s0, gtiles);
         auto cost_of = [&](int64_t c) { return ((ntiles * ((n + c - 1) / c) + cap - 1) / cap + lone) * (c + over); };
         int64_t best = cost_of(chunk);  // the base plan stays unless a candidate beats it
         for (int64_t s = std::max<int64_t>(1, s0 / 2); s <= smax; s += s < 8 || nr > 1 ? 1 : 8) {
