@@ -175,9 +175,30 @@ constexpr size_t kSymSmallBytes = size_t(512) << 20;
 //                         24,000: 214 / 188 / 216    63,480: 1125 / 1171 / 1463
 //   2D Helmholtz CF FP64   6,006: 333 / - / 179 (328)  30,720: 2592 / - / 2583
 //   2D Helmholtz CF mixed  6,006: 123 / - / 82 (146)   40,000: 1989 / - / 2019
+// Where the 256-node tile pairs nearly fill their last round (4 blocks per CU) the
+// smaller tiles of the cheap pairs gain nothing and cost their staging: there
+// 3D Laplace but for SL, from about 15,400 nodes, keeps 256 nodes, and so do mixed
+// 2D Laplace DL (29,000), mixed Laplace SL and 2D (38,000) and, in the two rounds
+// that end at 16,128 nodes, 2D Laplace but for the logarithms and mixed 3D
+// Helmholtz SL and CF. With 256 / 128 at full rounds: 16,125 nodes, 2D Laplace DL
+// mixed 0.88x, HS 0.90x; 3D Laplace HS FP64 0.92x, mixed 3D Helmholtz SL 0.93x;
+// 28,000: mixed 3D Laplace DL 268 / 289 us, FP64 346 / 381; 46,077: mixed 2D
+// Laplace DL 0.94x; with rounds 0.8 - 0.9 full (21,245, 26,877 nodes) 128 nodes
+// are up to 9 % faster.
 // Sums of 256 nodes or fewer run in one direction (k_apply_row). An explicit
 // group has tiles of 256. Beyond kSymMaxBytes of partial sums the groups of
 // 2 and 4 tiles halve and quarter them.
+static bool full_rounds(const Op *op, int kind, int64_t blocks) {
+    const int64_t cu = op->ctx->num_cu, round = 4 * cu, rounds = (blocks + round - 1) / round;
+    if ((double)blocks < 0.93 * (double)(rounds * round)) return false;
+    const bool mixed = op->precision == INTI_MIXED, two = rounds == 2, sl = kind == INTI_SL;
+    const bool dl = kind == INTI_DL || kind == INTI_ADL;
+    if (op->pde == INTI_HELMHOLTZ) return two && mixed && (sl || kind == INTI_COMB_SD);
+    if (op->dim == 3) return sl ? mixed && blocks >= 44 * cu : rounds >= 2;
+    if (mixed && blocks >= (dl ? 26 : 44) * cu) return true;
+    return two && !sl && (mixed || kind != INTI_COMB_SD);
+}
+
 bool plan_sym(const Op *op, int kind, SymPlan &P) {
     if (op->sym == 0 || op->trg != op->src || kind >= INTI_FF_SL || op->kimag != 0.0) return false;
     const int64_t n = op->src->n;
@@ -199,7 +220,7 @@ bool plan_sym(const Op *op, int kind, SymPlan &P) {
         const bool mixed = op->precision == INTI_MIXED;
         if (helm2 ? !mixed || t256 * (t256 + 1) / 2 < 24 * cu : t128 * (t128 + 1) / 2 < 12 * cu) tile = 64;
         else if (helm2) tile = kSymBS;
-        else if (t256 * (t256 + 1) / 2 < 72 * cu) tile = 128;
+        else if (t256 * (t256 + 1) / 2 < 72 * cu) tile = full_rounds(op, kind, t256 * (t256 + 1) / 2) ? kSymBS : 128;
         if (tile < kSymBS && (size_t)tiles(tile) * (size_t)n * es <= kSymSmallBytes) {
             P = SymPlan{tile, 1, tiles(tile), tiles(tile)};
             return true;

@@ -219,3 +219,12 @@ def test_more_targets_than_a_launch_of_64_threads_each(inti):
     ref = inti.IntegralOperator(K, inti.points(np.ascontiguousarray(X[:, rows])), Q) @ x
     say(f"[gpu] {m} targets: {np.linalg.norm(y - ref) / np.linalg.norm(ref):.2e}")
     assert np.linalg.norm(y - ref) <= 1e-13 * np.linalg.norm(ref)
+
+
+# both sides of the rounds of 256-node tile pairs that some kinds keep
+@pytest.mark.parametrize("pde,dim,kind", [(0, 2, 1), (0, 3, 3), (1, 3, 0), (0, 2, 0)])
+@pytest.mark.parametrize("n", [16128, 16129, 25599])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_full_rounds(inti, oracle, pde, dim, kind, n, precision):
+    Q = _nodes(inti, dim, n)
+    _check(inti, oracle, pde, dim, kind, Q, Q, precision)
