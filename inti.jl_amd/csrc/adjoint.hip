@@ -937,7 +937,6 @@ static int adjoint_sigma_only(Op *op, const double *ubar, double *sigma_bar) {
     for (int64_t i = 0; i < m; ++i) hc[i] = cplx ? make_double2(ubar[2 * i], -ubar[2 * i + 1]) : make_double2(ubar[i], 0.0);
     std::vector<double> hx;
     if (!cplx) hx.assign(ubar, ubar + m);
-    if (int rc = op_transpose_correction(op)) return rc;
     double2 *dc;
     double *dx, *dpart, *dsb;
     Arena mem(ctx);
@@ -1085,8 +1084,6 @@ int op_adjoint(Op *op, const double *ubar, const double *sigma, double *sigma_ba
     // gradient: the symmetric pass sums the two parts, the two-pass path adds
     // the target part on the host
     std::vector<double> kp(nsb), xsep(comb && !fsym ? (size_t)dim * m : 0);
-    if (sigma_bar)
-        if (int rc = op_transpose_correction(op)) return rc;
     double2 *dc, *dsg;
     double *dpart, *dsb, *dyb, *dnb, *dwb, *dkp, *dxb;
     Arena mem(ctx);

@@ -77,7 +77,7 @@ struct Op {
     double cid[2] = {0, 0};          // identity coefficient (square ops)
     const Quad *trg = nullptr, *src = nullptr;
     Csr *corr = nullptr;  // owned merged correction (may be null)
-    // the correction's transposed pattern (built by the first pullback; the
+    // the correction's transposed pattern (built at the first attach; the
     // pattern never changes while attached): column j's entries are
     // corr_trow[p] / corr->val[corr_tperm[p]] for p in [corr_tptr[j],
     // corr_tptr[j+1]), rows increasing. The adjoint gathers through it.
@@ -160,7 +160,6 @@ int refine_solve(Op *op_hi, Op *op_lo, Op *prec, const double *b, double *x, int
                  double *relres);
 int launch_assemble(const Op *op, double *out_dev);
 void op_free_correction(Op *op);
-int op_transpose_correction(Op *op);  // builds corr_tptr ... once
 int op_adjoint(Op *op, const double *ubar, const double *sigma, double *sigma_bar, double *ybar,
                double *nbar, double *wbar, double *xbar, const double *dcoefs, double *kbar);
 
