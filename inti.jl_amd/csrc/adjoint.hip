@@ -847,26 +847,50 @@ void plan(int64_t own, int64_t inner, int num_cu, int &split, int64_t &chunk) {
 }  // namespace
 
 // sigma_bar_j = conj(w_j post z_j) (complex) or w_j post z_j (real), z the
-// transposed sum's S partial slots added in slot order
+// transposed sum's S partial slots. NS = 4: the four waves of a block share the
+// slots of 64 nodes in contiguous quarters, added in wave order (one thread per
+// node waits on its chain of S loads, 18 us for the 68 slots of 4,320 nodes:
+// whole calls, 3D Helmholtz CF, 4,320 nodes 98 -> 83 us, 2D Laplace DL, 7,900:
+// 123 -> 96).
+template <int NS>
 __global__ __launch_bounds__(256) void k_adj_trans_reduce(int64_t n, int64_t S, int cplx, const double *part,
                                                           double pr, double pi, const double *w, double *sb) {
-    const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (j >= n) return;
+    constexpr int ROWS = 256 / NS;
+    __shared__ double2 s_w[NS][ROWS];
+    const int row = threadIdx.x % ROWS, share = threadIdx.x / ROWS;
+    const int64_t j = (int64_t)blockIdx.x * ROWS + row, jc = j < n ? j : n - 1;
+    const int64_t per = (S + NS - 1) / NS, q0 = share * per, q1 = q0 + per < S ? q0 + per : S;
+    double zr = 0.0, zi = 0.0;
     if (cplx) {
         const double2 *pp = reinterpret_cast<const double2 *>(part);
-        double zr = 0.0, zi = 0.0;
-        for (int64_t q = 0; q < S; ++q) {
-            const double2 v = pp[q * n + j];
+#pragma unroll 8
+        for (int64_t q = q0; q < q1; ++q) {
+            const double2 v = pp[q * n + jc];
             zr += v.x;
             zi += v.y;
         }
-        const double wj = w[j];
+    } else {
+#pragma unroll 8
+        for (int64_t q = q0; q < q1; ++q) zr += part[q * n + jc];
+    }
+    if constexpr (NS > 1) {
+        s_w[share][row] = make_double2(zr, zi);
+        __syncthreads();
+    }
+    if (share || j >= n) return;
+    if constexpr (NS > 1) {
+#pragma unroll
+        for (int t = 1; t < NS; ++t) {
+            zr += s_w[t][row].x;
+            zi += s_w[t][row].y;
+        }
+    }
+    const double wj = w[j];
+    if (cplx) {
         sb[2 * j] = wj * (pr * zr - pi * zi);
         sb[2 * j + 1] = -wj * (pr * zi + pi * zr);
     } else {
-        double z = 0.0;
-        for (int64_t q = 0; q < S; ++q) z += part[q * n + j];
-        sb[j] = w[j] * pr * z;
+        sb[j] = wj * pr * zr;
     }
 }
 
@@ -973,8 +997,14 @@ static int adjoint_sigma_only(Op *op, const double *ubar, double *sigma_bar) {
     }
     INTI_HIP(ctx, hipGetLastError());
     if (ctx->profiling) INTI_HIP(ctx, hipEventRecord(ctx->ev1, s));
-    hipLaunchKernelGGL(k_adj_trans_reduce, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, S, cplx,
-                       dpart, kp.postr, kp.posti, op->src->weights, dsb);
+    // four waves per 64 nodes where blocks of 256 would leave CUs idle, as in the
+    // forward sum's reduction
+    if (S >= 16 && (n + 255) / 256 < ctx->num_cu)
+        hipLaunchKernelGGL(k_adj_trans_reduce<4>, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, s, n, S, cplx, dpart,
+                           kp.postr, kp.posti, op->src->weights, dsb);
+    else
+        hipLaunchKernelGGL(k_adj_trans_reduce<1>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, S, cplx, dpart,
+                           kp.postr, kp.posti, op->src->weights, dsb);
     INTI_HIP(ctx, hipGetLastError());
     if (op->corr) {
         hipLaunchKernelGGL(k_adj_corr, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, op->corr_tptr,

@@ -42,3 +42,28 @@ def test_tiles_match_two_passes(inti, pde, dim, kind, n, comb):
             size = max(size, np.linalg.norm(u) * np.linalg.norm(x) / n)
         print(f"[gpu] pde {pde} dim {dim} {kind} n={n} {key}: {err:.2e} of {size:.2e}", flush=True)
         assert err <= 1e-11 * size
+
+
+@pytest.mark.parametrize("pde,dim,kind", [(0, 2, "DL"), (0, 3, "SL"), (0, 3, "DL"), (1, 2, "CF"), (1, 3, "SL"), (1, 3, "CF")])
+@pytest.mark.parametrize("n,mode,group", [(700, 2, 0), (700, 2, 1), (700, 2, 2), (1300, 2, 4), (1025, 1, 0), (7900, 1, 0),
+                                          (10001, 1, 0), (10001, 2, 2), (49409, 1, 0), (66000, 1, 0)])
+def test_sigma_only_tiles(inti, pde, dim, kind, n, mode, group):
+    """sigma-bar alone, A^H ubar, by the transposed symmetric sum: 64-node tiles
+    (small n), 128 (10,001), 256 (explicit groups, and 49,409 nodes up) and both
+    forms of its reduction (16 slots, 65,536 nodes), against the one-direction
+    sum, to 1e-12 of its size (FP64 sums of n terms of one size in another order:
+    sqrt(66,000) 2^-53 = 3e-14)."""
+    Q = _nodes(inti, dim, n)
+    op = inti.Helmholtz(k=4.1, dim=dim) if pde else inti.Laplace(dim=dim)
+    K = {"SL": inti.SingleLayerKernel, "DL": inti.DoubleLayerKernel}[kind](op) if kind != "CF" else \
+        inti.CombinedFieldKernel(op, -4.1j, 1.0, "SD")
+    rng = np.random.default_rng(6)
+    x, u = (rng.normal(size=n) + (1j * rng.normal(size=n) if pde else 0.0) for _ in range(2))
+    out = {}
+    for m, g in ((0, 0), (mode, group)):
+        A = inti.IntegralOperator(K, Q, Q)
+        A.set_symmetric(m, g)
+        out[m] = A.pullback(u, x, wrt=("sigma",))["sigma"]
+    err, size = np.linalg.norm(out[mode] - out[0]), np.linalg.norm(out[0])
+    print(f"[gpu] sigma-bar pde {pde} dim {dim} {kind} n={n} mode {mode} group {group}: {err:.2e} of {size:.2e}", flush=True)
+    assert err <= 1e-12 * size
