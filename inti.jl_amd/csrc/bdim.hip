@@ -154,7 +154,15 @@ __device__ __forceinline__ void theta_pair(const double *r, const double *nx, co
         helm2_combine<KS, false>(r, ok, nx, ny, p, R, sr, si);
         helm2_combine<KD, false>(r, ok, nx, ny, p, R, dr, di);
     } else {
-        pair_raw<PDE, DIM, KS, false>(r, nx, ny, p, sr, si);
+        if constexpr (PDE == INTI_LAPLACE && DIM == 2 && KS == INTI_SL) {
+            // the library's logarithm, as in the traces and mu G that Theta
+            // cancels against (pair_value)
+            const double d2 = dotv<2>(r, r);
+            sr = mask(d2 > kSamePointTol2, log(fmax(d2, kClampD2)));
+            si = 0.0;
+        } else {
+            pair_raw<PDE, DIM, KS, false>(r, nx, ny, p, sr, si);
+        }
         pair_raw<PDE, DIM, KD, false>(r, nx, ny, p, dr, di);
     }
 }
