@@ -104,11 +104,34 @@ void op_free_correction(Op *op) {
 }
 
 // Transposed pattern of an attached correction for the adjoint's gather (rows
-// increasing within a column), built on the GPU by the attach: entries counted
-// per column, the counts summed, entries dropped into their columns in any
-// order, and each column sorted by its entries' positions in the CSR. The host's
-// counting sort took 280 us of an attach at 12,000 nodes (63,480: 700); these
-// kernels take 35 (50).
+// increasing within a column), built on the GPU by the attach. A pattern equal to
+// its transpose (each element's own nodes) takes one kernel, which looks up entry
+// (j, i) in row j for every (i, j) and sets *flag where it is missing; any other
+// is sorted: entries counted per column, the counts summed, entries dropped into
+// their columns in any order, and each column sorted by its entries' positions in
+// the CSR. The host's counting sort took 280 us of an attach at 12,000 nodes
+// (63,480: 700); the one kernel adds 9 (10), the sort's five 35 (50).
+constexpr int64_t kOwnRow = 32;  // average entries per row up to which the lookup is tried
+
+__global__ __launch_bounds__(256) void k_own_transpose(int64_t n, const int32_t *rowptr, const int32_t *colind,
+                                                       int32_t *tptr, int32_t *trow, int32_t *tperm, int *flag) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const int32_t p0 = rowptr[i], p1 = rowptr[i + 1];
+    tptr[i] = p0;
+    if (i == n - 1) tptr[n] = p1;
+    bool bad = false;
+    for (int32_t p = p0; p < p1; ++p) {
+        const int32_t j = colind[p], q1 = rowptr[j + 1];
+        int32_t q = rowptr[j];
+        while (q < q1 && colind[q] != (int32_t)i) ++q;
+        bad |= q == q1 || (p > p0 && colind[p - 1] >= j);
+        trow[p] = j;
+        tperm[p] = q;
+    }
+    if (bad) *flag = 1;
+}
+
 __global__ __launch_bounds__(256) void k_col_count(int64_t nnz, const int32_t *colind, int32_t *count) {
     const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (q < nnz) atomicAdd(&count[colind[q]], 1);
@@ -219,24 +242,31 @@ __global__ __launch_bounds__(256) void k_col_sort(int64_t n, const int32_t *tptr
     }
 }
 
-// on ctx->stream, not waited for
-static int transpose_pattern(Op *op) {
+// The pattern of op->corr transposed: enqueued on ctx->stream; with `own` the
+// lookup, whose *ctx->flag the caller reads after its wait, else the sort
+static int transpose_pattern(Op *op, bool own) {
     Ctx *ctx = op->ctx;
     const Csr *c = op->corr;
-    const int64_t m = c->m, n = c->n, nnz = c->nnz;
+    const int64_t m = c->m, n = c->n, nnz = c->nnz, nb = (n + 1023) / 1024;
     const size_t ib = sizeof(int32_t), most = std::max<size_t>((size_t)nnz, 1);
-    const int64_t nb = (n + 1023) / 1024;
-    void *scr = nullptr;
-    if (int st = ctx_scratch(ctx, kScrArena, ib * (size_t)(n + nb), &scr)) return st;
-    int32_t *fill = (int32_t *)scr, *sums = fill + n;
-    if (hipMalloc((void **)&op->corr_tptr, ib * ((size_t)(n + 1) + 2 * most)) != hipSuccess) {
+    if (!op->corr_tptr && hipMalloc((void **)&op->corr_tptr, ib * ((size_t)(n + 1) + 2 * most)) != hipSuccess) {
         op->corr_tptr = nullptr;
         return set_error(ctx, INTI_ERR_NOMEM, "attach: transposed pattern allocation failed");
     }
     op->corr_trow = op->corr_tptr + n + 1;
     op->corr_tperm = op->corr_trow + most;
-    hipStream_t s = ctx->stream;
     if (n == 0) return INTI_OK;  // no column to read
+    hipStream_t s = ctx->stream;
+    if (own) {
+        *ctx->flag = 0;
+        hipLaunchKernelGGL(k_own_transpose, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, c->rowptr, c->colind,
+                           op->corr_tptr, op->corr_trow, op->corr_tperm, ctx->flag);
+        INTI_HIP(ctx, hipGetLastError());
+        return INTI_OK;
+    }
+    void *scr = nullptr;
+    if (int st = ctx_scratch(ctx, kScrArena, ib * (size_t)(n + nb), &scr)) return st;
+    int32_t *fill = (int32_t *)scr, *sums = fill + n;
     INTI_HIP(ctx, hipMemsetAsync(fill, 0, ib * (size_t)n, s));
     if (nnz > 0)
         hipLaunchKernelGGL(k_col_count, dim3((unsigned)((nnz + 255) / 256)), dim3(256), 0, s, nnz, c->colind, fill);
@@ -441,7 +471,8 @@ int inti_ctx_create(int device, inti_ctx **out) {
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) == hipSuccess) c->num_cu = prop.multiProcessorCount;
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess) {
+        hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess ||
+        hipHostMalloc((void **)&c->flag, sizeof(int), hipHostMallocMapped) != hipSuccess) {
         delete c;
         return set_error(nullptr, INTI_ERR_HIP, "stream/event creation failed");
     }
@@ -450,6 +481,7 @@ int inti_ctx_create(int device, inti_ctx **out) {
     void *sp = nullptr;
     const hipError_t se = hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch));
     if (se != hipSuccess || sp == nullptr) {
+        (void)hipHostFree(c->flag);
         (void)hipEventDestroy(c->ev0);
         (void)hipEventDestroy(c->ev1);
         (void)hipStreamDestroy(c->stream);
@@ -467,6 +499,7 @@ int inti_ctx_destroy(inti_ctx *ctx) {
     (void)hipStreamSynchronize(ctx->stream);
     for (int s = 0; s < Ctx::kSlots; ++s)
         if (ctx->scratch[s]) (void)hipFree(ctx->scratch[s]);
+    (void)hipHostFree(ctx->flag);
     (void)hipEventDestroy(ctx->ev0);
     (void)hipEventDestroy(ctx->ev1);
     (void)hipStreamDestroy(ctx->stream);
@@ -905,23 +938,19 @@ int inti_op_attach_correction(inti_op *op, const inti_csr *csr, double coef_re, 
     LOCK(ctx);
     const int cplx = csr->is_complex;
     int accumulate = 0;
+    bool own = false;
     if (op->corr) {
         // same pattern required for an in-place merge
         bool same = op->corr->nnz == csr->nnz;
         if (same && csr->nnz > 0) {
-            int differ = 0, *dflag = nullptr;
-            void *scr = nullptr;
-            if (int st = ctx_scratch(ctx, kScrArena, sizeof(int), &scr)) return st;
-            dflag = (int *)scr;
-            INTI_HIP(ctx, hipMemcpyAsync(dflag, &differ, sizeof(int), hipMemcpyHostToDevice, ctx->stream));
+            *ctx->flag = 0;
             hipLaunchKernelGGL(k_differ, dim3((unsigned)((csr->m + 256) / 256)), dim3(256), 0, ctx->stream, csr->m + 1,
-                               op->corr->rowptr, csr->rowptr, dflag);
+                               op->corr->rowptr, csr->rowptr, ctx->flag);
             hipLaunchKernelGGL(k_differ, dim3((unsigned)((csr->nnz + 255) / 256)), dim3(256), 0, ctx->stream, csr->nnz,
-                               op->corr->colind, csr->colind, dflag);
+                               op->corr->colind, csr->colind, ctx->flag);
             INTI_HIP(ctx, hipGetLastError());
-            INTI_HIP(ctx, hipMemcpyAsync(&differ, dflag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
             INTI_HIP(ctx, hipStreamSynchronize(ctx->stream));
-            same = differ == 0;
+            same = *ctx->flag == 0;
         }
         if (!same)
             return set_error(ctx, INTI_ERR_UNSUPPORTED, "attach: corrections with different patterns cannot be merged");
@@ -934,7 +963,8 @@ int inti_op_attach_correction(inti_op *op, const inti_csr *csr, double coef_re, 
         INTI_HIP(ctx, hipMemcpyAsync(c->rowptr, csr->rowptr, sizeof(int32_t) * (csr->m + 1), hipMemcpyDeviceToDevice, ctx->stream));
         if (csr->nnz > 0)
             INTI_HIP(ctx, hipMemcpyAsync(c->colind, csr->colind, sizeof(int32_t) * csr->nnz, hipMemcpyDeviceToDevice, ctx->stream));
-        st = transpose_pattern(op);
+        own = csr->m == csr->n && csr->nnz <= kOwnRow * csr->m;
+        st = transpose_pattern(op, own);
         if (st) {
             (void)hipStreamSynchronize(ctx->stream);
             op_free_correction(op);
@@ -947,6 +977,13 @@ int inti_op_attach_correction(inti_op *op, const inti_csr *csr, double coef_re, 
         INTI_HIP(ctx, hipGetLastError());
     }
     INTI_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (own && *ctx->flag) {
+        if (int st = transpose_pattern(op, false)) {
+            (void)hipStreamSynchronize(ctx->stream);
+            op_free_correction(op);
+            return st;
+        }
+    }
     return INTI_OK;
 }
 

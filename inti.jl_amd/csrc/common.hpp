@@ -40,6 +40,9 @@ struct Ctx {
     // device address of the library's static partial-sum buffer on this
     // context's device (the allocation-free apply)
     double *noalloc_scratch = nullptr;
+    // pinned host memory that kernels set and the host reads after its wait
+    // (under mu): the answer of a yes / no kernel without a copy each way
+    int *flag = nullptr;
 };
 
 struct Quad {

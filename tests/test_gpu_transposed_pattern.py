@@ -1,6 +1,7 @@
 """The transposed pattern of an attached correction (built on the GPU by the
-attach) through sigma-bar = A^H ubar: corrections of each element's own nodes,
-of all targets for every element (columns of every length up to all rows), and
+attach) through sigma-bar = A^H ubar: corrections of each element's own nodes (a
+pattern that is its own transpose), of these and twenty more targets for one
+element (nearly so: the lookup finds an entry missing and the sort runs), of all targets for every element (columns of every length up to all rows), and
 of all targets for a few elements only (long and short columns, some empty).
 Against the dense matrix's conjugate transpose (1e-12: sums of a few hundred
 terms), twice attached, and bit-identical for two operators. The first pullback
@@ -19,7 +20,7 @@ def _near(n, ne, lists):
 
 
 @pytest.mark.parametrize("pde", [0, 1])
-@pytest.mark.parametrize("pattern", ["own", "all", "few", "targets"])
+@pytest.mark.parametrize("pattern", ["own", "lopsided", "all", "few", "targets"])
 def test_sigma_bar(inti, pde, pattern):
     Q = inti.sphere_quadrature(2, qorder=4)
     n, ne = len(Q), Q.ne
@@ -28,7 +29,8 @@ def test_sigma_bar(inti, pde, pattern):
         if pattern == "targets" else Q
     m = len(T)
     every, own = np.arange(m), [np.sort(Q.qtags[:, e]) for e in range(ne)]
-    near = {"own": None, "all": _near(n, ne, [every] * ne),
+    near = {"own": None, "lopsided": _near(n, ne, [np.union1d(own[e], every[100:120]) if e == 70 else own[e] for e in range(ne)]),
+            "all": _near(n, ne, [every] * ne),
             "few": _near(n, ne, [every if e % 7 == 3 else own[e] if e % 7 < 3 else own[0][:0] for e in range(ne)]),
             "targets": _near(n, ne, [every[e % 3::3] if e < 60 else every[:0] for e in range(ne)])}[pattern]
     S, D = (inti.IntegralOperator(K(op), T, Q) for K in (inti.SingleLayerKernel, inti.DoubleLayerKernel))
