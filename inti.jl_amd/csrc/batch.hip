@@ -87,6 +87,9 @@ static BatchFn pick_batch(int pde, int dim, int kind, int mixed, int nr) {
 // 230 / 340 / 500; 12 of 17,328: 187 / 225 / 257 / 461; 3 of 1,884: 72 / 127 /
 // 180 / 278; 200 of 325,424: 3264 / 3166 / 3148 / 3213 (FP64 6617 / 6635 /
 // 6728 / 6873).
+// One and four densities follow the same rule: against 2048, mixed, 48 problems
+// of 79,088 nodes 788 -> 543 and 963 -> 669, of 37,824: 464 -> 143 and 549 -> 172,
+// 3 of 1,884: 324 -> 75 and 369 -> 85, 200 of 325,424 unchanged.
 static int64_t batch_chunk(const Batch *B) {
     const int64_t slots = 2LL * B->ctx->num_cu;
     auto plan = [&](int64_t L, int64_t &items, int64_t &sums) {

@@ -18,6 +18,10 @@
 // the same order), updates its rows and forms the next pass's partial dots or
 // norm while the rows are in LDS. (Ten kernels before, each with its own
 // sweep: GMRES on 4,320 complex nodes 2.58 -> 1.97 ms.)
+// The redundant sums grow with the columns as the sweeps over the basis do, and
+// stay below them also at 16,384 nodes, the most blocks per row (256 blocks of 64
+// rows): 500 / 2,000 / 5,000 steps of one basis take 0.26 / 1.36 / 6.8 s, with
+// the ten kernels 0.39 / 2.93 / 16.5 s.
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
